@@ -185,9 +185,10 @@ __device__ __forceinline__ void emit_split_run(std::uint64_t r, const float (&v)
     const std::uint32_t g = static_cast<std::uint32_t>(r & 3u);
     half8v hi, lo;
     split8(v, s, hi, lo);
-    float sum = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) sum += v[e] * s;
+    // As a tree: a Q4_K product leans on this sum (offset times sum against
+    // codes times values), and its rounding is common to every output.
+    float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    sum *= s;
     sum += __shfl_xor(sum, 1);
     sum += __shfl_xor(sum, 2);
     const std::uint32_t lane = (m & 15u) + 16u * g;

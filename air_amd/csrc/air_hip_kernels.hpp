@@ -249,6 +249,7 @@ struct SkinnyShape {
     std::uint32_t splits{1};
     std::uint32_t lds_stages{0};  // Q8_0 from split activations: stages of the LDS pipeline (0 = registers)
     std::uint32_t waves{4};       // waves per workgroup: 4, or 8 on the LDS pipeline
+    bool stream{false};           // the streaming kernel (linear_stream.hip): waves 8 or 10
 };
 // lds_stages: 0 automatic, 1 the register pipeline, 2..4 the LDS ring
 // (Q8_0 from split activations; other formats and f32 inputs ignore it).
@@ -263,6 +264,14 @@ std::uint64_t skinny_partials_bytes(const SkinnyShape& shape, std::uint32_t m, s
 // launches) combines a K split inside the kernel instead of a reduction
 // launch, with the reduction's bits.
 hipError_t launch_skinny_linear(const TilePlanes& planes, const SplitWorkspace& ws, const float* bias, float* y,
+                                std::uint32_t m, const SkinnyShape& shape, float* partials, hipStream_t stream,
+                                const SplitEpilogue* epilogue = nullptr, std::uint64_t* chain = nullptr);
+// The streaming kernel (linear_stream.hip) over the same split activations:
+// whether the automatic route takes it for m rows, its plan (shape.stream), and
+// the launch (launch_skinny_linear calls it for such a shape).
+bool stream_preferred(const TilePlanes& planes, std::uint32_t m);
+SkinnyShape plan_stream(const TilePlanes& planes, std::uint32_t m);
+hipError_t launch_stream_linear(const TilePlanes& planes, const SplitWorkspace& ws, const float* bias, float* y,
                                 std::uint32_t m, const SkinnyShape& shape, float* partials, hipStream_t stream,
                                 const SplitEpilogue* epilogue = nullptr, std::uint64_t* chain = nullptr);
 // The same linear straight from f32 activations x [m][k]: each workgroup

@@ -351,6 +351,22 @@ bool dense_prefill(const air_hip_context* ctx, const air_hip_matrix* m, std::uin
 // the launch path and for air_hip_linear_plan.
 enum class Route { prefill, gemv, fused, skinny_x, skinny_loaded, decode_linear, dense, wsplit };
 
+// No override of the 2..64-row decode kernels is set: each asks for a kernel
+// of its own, and the streaming kernel has none.
+bool decode_automatic(const air_hip_context* ctx) {
+    const WsplitTuning& w = ctx->wsplit_tuning;
+    return ctx->decode_path == 0u && ctx->wsplit_mode == 0u && ctx->skinny_tile_n == 0u && ctx->skinny_splits == 0u &&
+           ctx->skinny_lds_stages == 0u && ctx->skinny_waves == 0u && w.tile_n == 0u && w.waves == 0u &&
+           w.depth == 0u && w.k_splits == 0u && w.split_x == 0u;
+}
+
+// The plan of the kernels over split activations: the streaming kernel where
+// the automatic route prefers it, else a skinny kernel.
+SkinnyShape skinny_plan(const air_hip_context* ctx, const TilePlanes& p, std::uint32_t rows) {
+    if (decode_automatic(ctx) && stream_preferred(p, rows)) return plan_stream(p, rows);
+    return plan_skinny(p, rows, ctx->skinny_tile_n, ctx->skinny_splits, ctx->skinny_lds_stages, ctx->skinny_waves);
+}
+
 // The skinny kernel straight from the f32 rows, or over activations split
 // into the workspace first.  The in-workgroup split repeats the activation
 // split in every workgroup: it pays on narrow matrices, where the separate
@@ -358,8 +374,8 @@ enum class Route { prefill, gemv, fused, skinny_x, skinny_loaded, decode_linear,
 // faster), and loses on wide ones (gate|up, lm_head: up to 2x slower) and at
 // M = 64.  Q4_K with four activation tiles would also spill in it.
 Route skinny_route(const air_hip_context* ctx, const air_hip_matrix* m, std::uint32_t rows) {
-    const SkinnyShape shape = plan_skinny(m->planes, rows, ctx->skinny_tile_n, ctx->skinny_splits, ctx->skinny_lds_stages,
-                                          ctx->skinny_waves);
+    const SkinnyShape shape = skinny_plan(ctx, m->planes, rows);
+    if (shape.stream) return Route::skinny_loaded;
     // From 17 rows the split activations feed the LDS pipeline, which beats
     // the f32-input kernel on the narrow 7B matrices too, split launch
     // included (Q8_0, M = 32: q|k|v 18.4 -> 16.2 us, o 16.3 -> 14.7, down
@@ -377,6 +393,7 @@ Route route_linear(const air_hip_context* ctx, const air_hip_matrix* m, std::uin
         return Route::prefill;
     }
     if (rows == 1u) return Route::gemv;
+    if (decode_automatic(ctx) && stream_preferred(m->planes, rows)) return Route::skinny_loaded;
     if (rows <= AIR_HIP_MAX_DECODE_ROWS &&
         (ctx->wsplit_mode == 1u ||
          (ctx->wsplit_mode == 0u && ctx->decode_path == 0u && wsplit_preferred(m->planes, rows)))) {
@@ -403,8 +420,7 @@ Route route_linear(const air_hip_context* ctx, const air_hip_matrix* m, std::uin
 // (two with a K split), no activation workspace.
 int run_skinny_x(air_hip_context* ctx, const air_hip_matrix* m, const float* x, float* y, const float* bias,
                  std::uint32_t rows, const SplitEpilogue* epilogue, bool* applied, const void* ready) {
-    const SkinnyShape shape = plan_skinny(m->planes, rows, ctx->skinny_tile_n, ctx->skinny_splits, ctx->skinny_lds_stages,
-                                          ctx->skinny_waves);
+    const SkinnyShape shape = skinny_plan(ctx, m->planes, rows);
     if (skinny_route(ctx, m, rows) == Route::skinny_loaded) {
         int rc = load_activations_for(ctx, x, m->planes.k, rows, ready);
         if (rc != AIR_HIP_OK) return rc;
@@ -1174,8 +1190,7 @@ int linear_loaded(air_hip_context* ctx, const air_hip_matrix* m, float* y, const
         return fail(AIR_HIP_INVALID_STATE, "activations were loaded for another decode path; load them again");
     }
     if (skinny) {
-        const SkinnyShape shape = plan_skinny(m->planes, rows, ctx->skinny_tile_n, ctx->skinny_splits, ctx->skinny_lds_stages,
-                                          ctx->skinny_waves);
+        const SkinnyShape shape = skinny_plan(ctx, m->planes, rows);
         const std::uint64_t partial_bytes = skinny_partials_bytes(shape, rows, m->planes.n);
         if (partial_bytes > 0u) {
             const int rc = ensure_split_buffers(ctx, partial_bytes, 0u);
@@ -1356,8 +1371,13 @@ std::string describe_linear(const air_hip_context* ctx, const air_hip_matrix* m,
     case Route::skinny_x:
     case Route::skinny_loaded: {
         const bool loaded = route_linear(ctx, m, rows, tactic) == Route::skinny_loaded;
-        const SkinnyShape k = plan_skinny(m->planes, rows, ctx->skinny_tile_n, ctx->skinny_splits, ctx->skinny_lds_stages,
-                                          ctx->skinny_waves);
+        const SkinnyShape k = skinny_plan(ctx, m->planes, rows);
+        if (k.stream) {
+            std::snprintf(buf, sizeof buf, "split_rows_kernel + stream_kernel<%s> mt=%u tile_n=%u waves=%u+2 groups=%u "
+                          "splits=%u%s", fmt, k.mt, k.tile_n, k.waves, k.groups, k.splits,
+                          split_tail(ctx, k.splits, rows, m->planes.n));
+            break;
+        }
         const bool lds = loaded && k.lds_stages >= 2u;
         char stages[32] = "";
         if (lds) std::snprintf(stages, sizeof stages, " lds_stages=%u%s", k.lds_stages, k.waves == 8u ? " waves=8" : "");
@@ -1432,8 +1452,7 @@ int air_hip_linear_noalloc(air_hip_context* ctx, const air_hip_matrix* m, const 
     SkinnyShape shape{};
     WsplitShape wshape{};
     if (route == Route::skinny_x || route == Route::skinny_loaded) {
-        shape = plan_skinny(p, rows, ctx->skinny_tile_n, ctx->skinny_splits, ctx->skinny_lds_stages,
-                                          ctx->skinny_waves);
+        shape = skinny_plan(ctx, p, rows);
         partial_bytes = skinny_partials_bytes(shape, rows, p.n);
     }
     if (route == Route::wsplit) {

@@ -792,6 +792,7 @@ std::uint64_t skinny_partials_bytes(const SkinnyShape& shape, std::uint32_t m, s
 hipError_t launch_skinny_linear(const TilePlanes& p, const SplitWorkspace& ws, const float* bias, float* y,
                                 std::uint32_t m, const SkinnyShape& shape, float* partials, hipStream_t stream,
                                 const SplitEpilogue* epilogue, std::uint64_t* chain) {
+    if (shape.stream) return launch_stream_linear(p, ws, bias, y, m, shape, partials, stream, epilogue, chain);
     if (m == 0u || m > 64u || shape.mt != ceil_div(m, 16u)) return hipErrorInvalidValue;
     SkinnyArgs a{};
     a.codes = p.codes;

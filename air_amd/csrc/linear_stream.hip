@@ -1,0 +1,554 @@
+// linear_stream.hip -- the decode linear for M = 2..64 rows over split
+// activations: weights streamed through registers, activations shared through
+// LDS by waves that do nothing else.
+//
+// The arithmetic of skinny_kernel / skinny_lds_kernel (linear_skinny.hip);
+// what differs is how the operands travel:
+//
+//   * a workgroup is W consumer waves that own W * TN 16-row weight tiles and
+//     every activation row, and kProducers waves; one workgroup per CU;
+//   * a consumer's codes and scales go straight to its registers, a ring of
+//     kRing records ahead of their use, with no barrier on their way; past
+//     the end of the range the loads repeat the last record (a cache hit)
+//     instead of branching, so the compiler's load counting stays exact and a
+//     wave waits for its oldest record only;
+//   * the producers move the activation fragments global -> LDS directly,
+//     chunks of kChunk steps, three ahead of the consumers.  Loads return in
+//     order: in one wave, every wait for a chunk of activations (L2) would
+//     also wait for the weights (HBM) asked for before it, and a pending
+//     direct load makes the compiler wait for every load before any register
+//     of one is read.  Staging by the consumers cost 9 us of gate|up at 32
+//     rows and 28 at 64 (7B, Q8_0, timed with the staging left out);
+//   * one bare barrier per chunk; a chunk's fragments are read from LDS one
+//     stage ahead of the MFMAs that use them;
+//   * the K sum is formed in levels where registers allow (kLevels): pairs
+//     of steps, trips of the ring, then the total.  One running sum of the
+//     112 blocks of K = 3584 is 2.3e-7 from 64 bits (relative L2, Q8_0), the
+//     kernels this one replaces, whose waves split K, 1.6e-7, this one 1.5e-7.
+//
+// What bounds it: HBM at one activation tile; at more, the L2 reads of the
+// activations (4 M K bytes per workgroup) and the LDS reads and VALU work per
+// weight tile, which grow with M.  Row tiles per workgroup are chosen so that
+// the grid is one round of the 256 CUs: a CU with two workgroups of eight
+// tiles finishes last (7B gate|up at 32 rows: 296 workgroups of eight tiles
+// 48 us, 237 of ten 36).
+//
+// Measured per linear (Qwen2-7B shapes, graph replay over copies larger than
+// the Infinity Cache, the split launch included; kernels replaced -> this):
+//
+//                 M = 8           16            32            64
+//   gate|up Q8_0  34.6 -> 30.4    37.8 -> 30.7  (kept)        64.9 -> 52.7 us
+//           Q4_0  33.8 -> 23.1    35.0 -> 23.2  45.2 -> 31.8  66.6 -> 51.0
+//           Q4_K  38.4 -> 28.1    38.3 -> 28.9  51.9 -> 40.0  78.1 -> 60.7
+//   down    Q8_0  -               -             36.3 -> 33.8  47.1 -> 39.9
+//           Q4_0  -               -             34.7 -> 29.6  45.2 -> 38.6
+//           Q4_K  31.1 -> 25.5    32.0 -> 26.4  40.1 -> 32.3  51.8 -> 44.1
+//   q|k|v   Q8_0  -               -             18.2 -> 16.9  23.5 -> 21.7
+//   lm_head Q8_0  121 -> 107      123 -> 108    140 -> 121    195 -> 191
+//           Q4_0  91 -> 73        92 -> 78      126 -> 107    197 -> 169
+//           Q4_K  115 -> 89       112 -> 90     158 -> 130    253 -> 206
+//
+// Replaces specialized_matmul_kernel / specialized_matmul_batch_reuse_kernel
+// (src/cuda/cuda_backend.cu:501-583) for batched decode.
+#include "air_hip_device.hpp"
+#include "air_hip_kernels.hpp"
+#include "air_hip_steps.hpp"
+
+#include <algorithm>
+#include <type_traits>
+#include <utility>
+
+namespace air_hip {
+namespace {
+
+struct StreamArgs {
+    const void* codes;
+    const void* scales;
+    std::uint32_t nt, kt;
+    std::uint64_t n;
+    const u32x4* xs;             // split activations [block][MT][2][64] x 16 B
+    std::uint32_t blocks;        // 32-element blocks of the workspace
+    const float* inv_scale;      // [mp] inverse power-of-two scale of each row
+    const float* block_sums;     // [block][mp] sums of the scaled values (Q4_K)
+    const float* bias;           // fused when not split over workgroups
+    float* out;                  // y, or partials [splits][m][n]
+    std::uint32_t m;
+    std::uint32_t groups;
+    std::uint32_t steps;
+    std::uint32_t steps_per_split;
+    std::uint32_t partial;
+    // K split combined in the kernel (chain_combine): slots [splits-1][m][n],
+    // y and the bias the last arrival adds; null: partials for a reduction.
+    std::uint64_t* chain;
+    float* y;
+    const float* chain_bias;
+    std::uint32_t splits;
+};
+
+typedef __attribute__((address_space(3))) void lds_void_t;
+typedef __attribute__((address_space(1))) void global_void_t;
+
+// Lane l's 16 (or 4) bytes land at lds_wave_base + l * 16 (l * 4).
+__device__ __forceinline__ void lds_load16(const void* src, void* lds_wave_base) {
+    __builtin_amdgcn_global_load_lds((global_void_t*)(const_cast<void*>(src)), (lds_void_t*)(lds_wave_base), 16, 0, 0);
+}
+__device__ __forceinline__ void lds_load4(const void* src, void* lds_wave_base) {
+    __builtin_amdgcn_global_load_lds((global_void_t*)(const_cast<void*>(src)), (lds_void_t*)(lds_wave_base), 4, 0, 0);
+}
+
+// s_waitcnt for vmcnt <= n only (expcnt and lgkmcnt at their maxima).
+template <unsigned n>
+__device__ __forceinline__ void wait_vm() {
+    static_assert(n < 64u, "vmcnt is six bits");
+    __builtin_amdgcn_s_waitcnt((n & 0xfu) | ((n >> 4) << 14) | (0x7u << 4) | (0xfu << 8));
+}
+
+// Workgroup barrier ordering LDS accesses only: loads in flight stay so.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <unsigned N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    [&]<std::size_t... I>(std::index_sequence<I...>) {
+        (f(std::integral_constant<unsigned, static_cast<unsigned>(I)>{}), ...);
+    }(std::make_index_sequence<N>{});
+}
+
+// A lane's share of one resident record of a row tile: kUnit steps of codes
+// and scales.
+template <int FMT>
+struct Record;
+template <>
+struct Record<kQ8_0> {
+    u32x4 c;
+    std::uint32_t d;
+};
+template <>
+struct Record<kQ4_0> {
+    u32x4 c;
+    u32x2 d;
+};
+template <>
+struct Record<kQ4_K> {
+    u32x4 c[2];
+    u32x4 h;
+};
+
+template <int FMT>
+constexpr unsigned kUnit = FMT == kQ8_0 ? 1u : FMT == kQ4_0 ? 2u : 4u;   // 64-k steps per record
+
+template <int FMT>
+__device__ __forceinline__ void load_record(const void* codes, const void* scales, std::uint64_t tile,
+                                            std::uint32_t lane, Record<FMT>& out) {
+    const u32x4* c = static_cast<const u32x4*>(codes);
+    if constexpr (FMT == kQ8_0) {
+        out.c = __builtin_nontemporal_load(c + tile * 64u + lane);
+        out.d = static_cast<const std::uint32_t*>(scales)[tile * 16u + (lane & 15u)];
+    } else if constexpr (FMT == kQ4_0) {
+        out.c = __builtin_nontemporal_load(c + tile * 64u + lane);
+        out.d = static_cast<const u32x2*>(scales)[tile * 16u + (lane & 15u)];
+    } else {
+        out.c[0] = __builtin_nontemporal_load(c + tile * 128u + lane);
+        out.c[1] = __builtin_nontemporal_load(c + tile * 128u + 64u + lane);
+        out.h = static_cast<const u32x4*>(scales)[tile * 16u + (lane & 15u)];
+    }
+}
+
+// Step `sub` (0 .. kUnit - 1) of a record as the step the shared decode reads.
+template <int FMT, unsigned sub>
+__device__ __forceinline__ StepCodes<FMT> record_step(const Record<FMT>& r) {
+    StepCodes<FMT> s;
+    if constexpr (FMT == kQ8_0) {
+        s.c = r.c;
+        s.d = r.d;
+    } else if constexpr (FMT == kQ4_0) {
+        s.c = sub == 0u ? u32x2{r.c.x, r.c.y} : u32x2{r.c.z, r.c.w};
+        s.d = sub == 0u ? r.d.x : r.d.y;
+    } else {
+        const u32x4 c = r.c[sub >> 1];
+        s.c = (sub & 1u) == 0u ? u32x2{c.x, c.y} : u32x2{c.z, c.w};
+        s.h = r.h;
+    }
+    return s;
+}
+
+// Steps per LDS chunk: kBuffers chunks of 4 C MT KiB are 128 KiB (96 with
+// three activation tiles), one workgroup per CU.
+template <int MT>
+constexpr unsigned kChunk = MT == 1 ? 8u : MT == 2 ? 4u : 2u;
+constexpr unsigned kBuffers = 4u;
+// Weight records in flight per wave: 8 KiB of codes (Q8_0), less where three
+// or four activation tiles need the registers.
+template <int FMT, int MT, int TN>
+constexpr unsigned kRing = FMT == kQ8_0   ? (MT <= 2 ? 8u : 4u) / TN
+                           : FMT == kQ4_0 ? (MT <= 2 && TN == 1 ? 4u : 2u)
+                                          : (TN == 1 ? 2u : 1u);
+constexpr int kProducers = 2;
+// Levels of the K sum: three, or as many as leave no register in scratch.
+template <int FMT, int MT, int TN>
+constexpr unsigned kLevels = MT <= 2 ? 3u : FMT == kQ4_K || (MT == 4 && TN == 2) ? 1u : 2u;
+
+template <int FMT, int MT, int TN, int W>
+__global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) void stream_kernel(StreamArgs a) {
+    constexpr unsigned P = kProducers;
+    constexpr unsigned U = kUnit<FMT>;
+    constexpr unsigned D = kRing<FMT, MT, TN>;
+    constexpr unsigned C = kChunk<MT>;
+    constexpr unsigned kBody = D * U > C ? D * U : C;       // steps per trip: the ring comes full circle
+    constexpr bool kSums = FMT == kQ4_K;
+    constexpr unsigned kMp = 16u * MT;
+    constexpr unsigned L = kLevels<FMT, MT, TN>;
+    constexpr unsigned kParts = MT <= 2 ? 2u : 1u;
+    constexpr unsigned kFrags = 2u * C * 2u * MT;           // 1 KiB activation fragments per chunk
+    constexpr unsigned kXBytes = kFrags * 1024u;
+    constexpr unsigned kSumLoads = kSums ? 2u * C * kMp / 64u : 0u;   // 64-float loads of a chunk's block sums
+    constexpr unsigned kChunkBytes = kXBytes + kSumLoads * 256u;
+    constexpr unsigned kXLoads = (kFrags + P - 1u) / P + (kSumLoads + P - 1u) / P;   // per producer and chunk
+    static_assert(kBody % C == 0u && kBody % (D * U) == 0u, "a trip is whole chunks and ring turns");
+    static_assert((kBuffers - 2u) * kXLoads < 64u, "vmcnt is six bits");
+    __shared__ __attribute__((aligned(1024))) unsigned char chunks[kBuffers * kChunkBytes];
+
+    const std::uint32_t lane = threadIdx.x & 63u;
+    const std::uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const std::uint32_t group = blockIdx.x % a.groups;
+    const std::uint32_t split = blockIdx.x / a.groups;
+    const std::uint32_t rt0 = (group * W + wave) * TN;
+    const std::uint32_t s_begin = split * a.steps_per_split;
+    const std::uint32_t s_end = min(a.steps, s_begin + a.steps_per_split);
+    const std::uint32_t chunk_count = (s_end - s_begin + C - 1u) / C;   // ranges are never empty
+
+    if (wave >= W) {
+        // Producer: fragment f of a chunk is block f / (2 MT) from its first,
+        // tile (f / 2) % MT, part f % 2; blocks past the workspace repeat the
+        // last one (not used), and so do loads past the chunk.
+        const std::uint32_t producer = wave - W;
+        const auto fill = [&](std::uint32_t c) __attribute__((always_inline)) {
+            unsigned char* base = chunks + (c % kBuffers) * kChunkBytes;
+            const std::uint32_t b0 = 2u * (s_begin + c * C);
+#pragma unroll
+            for (unsigned j = 0; j < (kFrags + P - 1u) / P; ++j) {
+                const unsigned f = min(producer + P * j, kFrags - 1u);
+                const std::uint32_t b = min(b0 + f / (2u * MT), a.blocks - 1u);
+                lds_load16(a.xs + (static_cast<std::uint64_t>(b) * (2u * MT) + f % (2u * MT)) * 64u + lane, base + f * 1024u);
+            }
+#pragma unroll
+            for (unsigned j = 0; j < (kSumLoads + P - 1u) / P; ++j) {
+                const unsigned q = min(producer + P * j, kSumLoads - 1u);
+                const unsigned e = q * 64u + lane;
+                const std::uint32_t b = min(b0 + e / kMp, a.blocks - 1u);
+                lds_load4(a.block_sums + static_cast<std::uint64_t>(b) * kMp + e % kMp, base + kXBytes + q * 256u);
+            }
+        };
+#pragma unroll
+        for (unsigned c = 0; c + 1u < kBuffers; ++c) fill(c);
+        for (std::uint32_t c = 0; c < chunk_count; ++c) {
+            wait_vm<(kBuffers - 2u) * kXLoads>();   // chunk c has landed
+            lds_barrier();                          // ... and chunk c - 1 is read
+            fill(c + kBuffers - 1u);
+        }
+        wait_vm<0u>();                              // nothing lands after the workgroup ends
+        return;
+    }
+
+    const std::uint32_t u_last = (s_end - 1u) / U;
+    float4v acc[TN][MT];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[j][t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+
+    float4v pair[L > 2u ? TN : 1][L > 2u ? MT : 1];   // the running pair of steps
+    float4v part[L > 1u ? TN : 1][L > 1u ? MT : 1];   // the running trip
+    // Tiles past the last row tile read the last one; they are not stored.
+    std::uint64_t wtile[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        wtile[j] = static_cast<std::uint64_t>(min(rt0 + static_cast<std::uint32_t>(j), a.nt - 1u)) * a.kt;
+    }
+    Record<FMT> ring[D][TN];
+    const auto load_w = [&](Record<FMT>(&dst)[TN], std::uint32_t unit) __attribute__((always_inline)) {
+        const std::uint32_t u = min(unit, u_last);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) load_record<FMT>(a.codes, a.scales, wtile[j] + u, lane, dst[j]);
+    };
+    // Stage q of a chunk (compile time): its fragments from LDS, read one
+    // stage ahead of the arithmetic so that no MFMA waits for an LDS read.  A
+    // stage is a block's two parts, or one of them (hi, then lo) with three
+    // or four activation tiles, whose registers hold no more.
+    half8v frag[2][MT][kParts];
+    float4v sums[kSums ? MT : 1];
+    const auto read_stage = [&]<unsigned q>(const unsigned char* base) __attribute__((always_inline)) {
+        constexpr unsigned blk = q * kParts / 2u;
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+#pragma unroll
+            for (unsigned i = 0; i < kParts; ++i) {
+                const unsigned f = (blk * MT + static_cast<unsigned>(t)) * 2u + (kParts == 2u ? i : q % 2u);
+                frag[q & 1u][t][i] = *reinterpret_cast<const half8v*>(base + f * 1024u + lane * 16u);
+            }
+        }
+    };
+    // The products of block `blk` of a chunk, block b of step `sub` of a
+    // record: every tile's high parts, then the low parts on top, so that
+    // neighbouring MFMAs do not depend on each other.  LAST: the chunk's last.
+    const auto compute = [&]<unsigned blk, unsigned sub, unsigned b, bool LAST>(
+                             const unsigned char* base, const Record<FMT>(&w_in)[TN]) __attribute__((always_inline)) {
+        constexpr unsigned q = blk * 2u / kParts;       // the block's first stage
+        half8v w[TN];
+        float ws[TN], wo[TN];
+        float4v p[TN][MT];
+        if constexpr (!LAST || kParts == 1u) read_stage.template operator()<q + 1u>(base);
+        const auto read_sums = [&]() __attribute__((always_inline)) {
+            if constexpr (kSums) {
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    sums[t] = *reinterpret_cast<const float4v*>(
+                        base + kXBytes + (blk * kMp + static_cast<unsigned>(t) * 16u + 4u * (lane >> 4)) * 4u);
+                }
+            }
+        };
+        if constexpr (kParts == 2u) read_sums();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const StepCodes<FMT> w_step = record_step<FMT, sub>(w_in[j]);
+            w[j] = step_codes<FMT>(w_step, b);
+            step_scale<FMT>(w_step, sub, b, ws[j], wo[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) p[j][t] = mfma16x16x32(frag[q & 1u][t][0], w[j], float4v{0.0f, 0.0f, 0.0f, 0.0f});
+        if constexpr (kParts == 1u) {
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!LAST) read_stage.template operator()<q + 2u>(base);
+            read_sums();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                p[j][t] = mfma16x16x32(kParts == 2u ? frag[q & 1u][t][kParts - 1u] : frag[(q + 1u) & 1u][t][0], w[j], p[j][t]);
+            }
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                float4v& sum = L > 2u ? pair[j][t] : L > 1u ? part[j][t] : acc[j][t];
+                if constexpr (L > 2u && blk % 4u == 0u) sum = ws[j] * p[j][t];
+                else sum += ws[j] * p[j][t];
+                if constexpr (kSums) sum -= wo[j] * sums[t];
+                if constexpr (L > 2u && blk % 4u == 3u) part[j][t] += sum;
+            }
+    };
+
+    // The weights' first records.
+    static_for<D>([&](auto d) __attribute__((always_inline)) {
+        load_w(ring[d.value], s_begin / U + d.value);
+        __builtin_amdgcn_sched_barrier(0);   // the loop's load counting needs this order too
+    });
+    // One trip: kBody steps from s.  WHOLE: all of them lie in the range.
+    std::uint32_t buffer = 0u;
+    const auto trip = [&](std::uint32_t s, auto whole_tag) __attribute__((always_inline)) {
+        constexpr bool WHOLE = decltype(whole_tag)::value;
+        bool done = false;
+        if constexpr (L > 1u) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) part[j][t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        const unsigned char* cur = chunks;
+        static_for<kBody>([&](auto i_tag) __attribute__((always_inline)) {
+            constexpr unsigned i = i_tag.value;
+            constexpr unsigned cs = i % C;                  // step of its chunk
+            if (!WHOLE && done) return;
+            if constexpr (cs == 0u) {
+                if (!WHOLE && i != 0u && s + i >= s_end) {
+                    done = true;
+                    return;
+                }
+                lds_barrier();
+                cur = chunks + buffer * kChunkBytes;
+                buffer = (buffer + 1u) % kBuffers;
+                read_stage.template operator()<0>(cur);
+            }
+            if (WHOLE || s + i < s_end) {
+                compute.template operator()<2u * cs, i % U, 0, false>(cur, ring[(i / U) % D]);
+                compute.template operator()<2u * cs + 1u, i % U, 1, cs + 1u == C>(cur, ring[(i / U) % D]);
+            }
+            if constexpr (i % U == U - 1u) load_w(ring[(i / U) % D], (s + i) / U + D);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        // A range that ends on the first step of a pair.
+        const bool open = L > 2u && !WHOLE && ((s_end - s_begin) & 1u) != 0u;
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                if constexpr (L > 2u) {
+                    if (open) part[j][t] += pair[j][t];
+                }
+                if constexpr (L > 1u) acc[j][t] += part[j][t];
+            }
+    };
+    std::uint32_t s = s_begin;
+    for (; s + kBody <= s_end; s += kBody) trip(s, std::true_type{});
+    if (s < s_end) trip(s, std::false_type{});
+
+    // D[row = activation row][col = weight row], as skinny_kernel.
+    float4v inv[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) inv[t] = reinterpret_cast<const float4v*>(a.inv_scale)[t * 4 + (lane >> 4)];
+    float* out = a.out + (a.partial ? static_cast<std::uint64_t>(split) * a.m * a.n : 0u);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const std::uint64_t n = static_cast<std::uint64_t>(rt0 + static_cast<std::uint32_t>(j)) * 16u + (lane & 15u);
+        if (rt0 + static_cast<std::uint32_t>(j) >= a.nt || n >= a.n) continue;
+        const float bn = a.bias ? a.bias[n] : 0.0f;
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const std::uint32_t m = static_cast<std::uint32_t>(t) * 16u + 4u * (lane >> 4) + static_cast<std::uint32_t>(i);
+                if (m >= a.m) continue;
+                const std::uint64_t e = static_cast<std::uint64_t>(m) * a.n + n;
+                float v = acc[j][t][i] * inv[t][i] + bn;
+                if (a.chain) {
+                    if (chain_combine(a.chain, static_cast<std::uint64_t>(a.m) * a.n, e, split, a.splits, v)) {
+                        a.y[e] = a.chain_bias ? v + a.chain_bias[n] : v;
+                    }
+                } else {
+                    out[e] = v;
+                }
+            }
+        }
+    }
+}
+
+template <int FMT, int MT, int TN, int W>
+hipError_t launch_w(const StreamArgs& a, std::uint32_t blocks, hipStream_t stream) {
+    hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W>), dim3(blocks), dim3(64 * (W + kProducers)), 0, stream, a);
+    return hipGetLastError();
+}
+
+template <int FMT, int MT>
+hipError_t launch_mt(const StreamArgs& a, const SkinnyShape& s, std::uint32_t blocks, hipStream_t stream) {
+    if (s.waves == 10u && s.tile_n == 2u) return launch_w<FMT, MT, 2, 10>(a, blocks, stream);
+    if (s.waves == 10u && s.tile_n == 1u) return launch_w<FMT, MT, 1, 10>(a, blocks, stream);
+    if (s.waves == 8u && s.tile_n == 1u) return launch_w<FMT, MT, 1, 8>(a, blocks, stream);
+    return hipErrorInvalidConfiguration;
+}
+
+template <int FMT>
+hipError_t launch_fmt(const StreamArgs& a, const SkinnyShape& s, std::uint32_t blocks, hipStream_t stream) {
+    switch (s.mt) {
+    case 1: return launch_mt<FMT, 1>(a, s, blocks, stream);
+    case 2: return launch_mt<FMT, 2>(a, s, blocks, stream);
+    case 3: return launch_mt<FMT, 3>(a, s, blocks, stream);
+    default: return launch_mt<FMT, 4>(a, s, blocks, stream);
+    }
+}
+
+} // namespace
+
+bool stream_preferred(const TilePlanes& p, std::uint32_t m) {
+    // Measured against the kernels it replaces on the Qwen2-7B matrices in all
+    // three formats at M = 3, 8, 16, 20, 32, 48 and 64 (graph replay, split
+    // launch included; the table at the top):
+    //  * wide matrices (over 1024 row tiles): faster at every width, but for
+    //    Q8_0 ones of 2000..4096 row tiles at 17..32 rows, whose eight-wave
+    //    plan and its two splits stay;
+    //  * narrow ones at two or more activation tiles: faster on q|k|v (1-2 us)
+    //    and, K being long, on down (2-9 us; Q8_0 from 25 rows: 33.3 against
+    //    32.6 us at 20); the matrices the wave-split kernel takes with short K
+    //    (o) keep it (16.5 against 14.5 us at 32 rows);
+    //  * narrow ones at one activation tile: only Q4_K with long K (down 31.1
+    //    -> 25.5 us at 8 rows; Q8_0 28.0 against 24.8, Q4_0 even).
+    // Short K (under 32 steps) leaves the ring and the chunks nothing to run
+    // ahead of, and under 96 row tiles the K splits that would fill the GPU
+    // cost more than they stream (33 tiles of K = 8448 at 6 rows: 23.6 us on
+    // the wave-split kernel, 31.6 here).
+    if (m < 2u || m > 64u || p.kp / kStepK < 32u) return false;
+    const bool one = m <= 16u, two = !one && m <= 32u;
+    if (p.nt > 1024u) return !(p.type == kQ8_0 && two && p.nt >= 2000u && p.nt <= 4096u);
+    if (p.nt < 96u) return false;
+    const bool long_k = p.k > 4096u;
+    if (one) return p.type == kQ4_K && long_k;
+    if (p.nt > 256u) return true;
+    if (p.type == kQ4_K && !two && p.k < 8192u) return false;   // even or slower at 33..64 rows (27.7, 28.2 us)
+    return long_k && (p.type != kQ8_0 || m > 24u);
+}
+
+SkinnyShape plan_stream(const TilePlanes& p, std::uint32_t m) {
+    SkinnyShape s;
+    s.stream = true;
+    s.mt = static_cast<std::uint32_t>(ceil_div(m, 16u));
+    s.steps = static_cast<std::uint32_t>(p.kp / kStepK);
+    // One round of 256 workgroups where the row tiles allow it: eight tiles a
+    // workgroup, ten from 2049 row tiles, twenty (two per wave, which also
+    // halves the activations read per tile: lm_head 141 -> 121 us at 32 rows)
+    // from 2561, where ten would start a second round.
+    s.tile_n = p.nt > 2560u ? 2u : 1u;
+    s.waves = p.nt > 2048u ? 10u : 8u;
+    s.groups = static_cast<std::uint32_t>(ceil_div(p.nt, s.waves * s.tile_n));
+    // Otherwise K is split over workgroups up to that round, at least twelve
+    // steps each (the partials' round trip: Q8_0 q|k|v at 32 rows 16.9 us with
+    // four splits, 17.6 with seven; ten with three or four activation tiles
+    // and eight for Q4_K, whose steps take longer: 18.4 and 17.3 us with four
+    // and six), and no further than plan_skinny would.
+    const std::uint32_t least = p.type == kQ4_K ? 8u : s.mt >= 3u ? 10u : 12u;
+    std::uint32_t splits = std::min(256u / std::min(s.groups, 256u), s.steps / least);
+    splits = std::min(splits, plan_skinny(p, m, 0u, 0u).splits);
+    splits = std::max(splits, 1u);
+    const std::uint32_t unit = p.type == kQ8_0 ? kUnit<kQ8_0> : p.type == kQ4_0 ? kUnit<kQ4_0> : kUnit<kQ4_K>;
+    s.steps_per_split = static_cast<std::uint32_t>(ceil_div(ceil_div(s.steps, splits), unit) * unit);
+    s.splits = static_cast<std::uint32_t>(ceil_div(s.steps, s.steps_per_split));
+    return s;
+}
+
+hipError_t launch_stream_linear(const TilePlanes& p, const SplitWorkspace& ws, const float* bias, float* y,
+                                std::uint32_t m, const SkinnyShape& shape, float* partials, hipStream_t stream,
+                                const SplitEpilogue* epilogue, std::uint64_t* chain) {
+    if (m == 0u || m > 64u || shape.mt != ceil_div(m, 16u) || shape.steps == 0u || shape.steps_per_split == 0u) {
+        return hipErrorInvalidValue;
+    }
+    StreamArgs a{};
+    a.codes = p.codes;
+    a.scales = p.scales;
+    a.nt = p.nt;
+    a.kt = p.kt;
+    a.n = p.n;
+    a.xs = static_cast<const u32x4*>(ws.xs);
+    a.blocks = static_cast<std::uint32_t>(p.kp / 32u);
+    a.inv_scale = ws.inv_scale;
+    a.block_sums = ws.block_sums;
+    a.m = m;
+    a.groups = shape.groups;
+    a.steps = shape.steps;
+    a.steps_per_split = shape.steps_per_split;
+    const bool split = shape.splits > 1u;
+    const bool chained = split && chain && !epilogue;
+    a.partial = split ? 1u : 0u;
+    a.bias = split ? nullptr : bias;
+    a.out = split ? partials : y;
+    if (chained) {
+        a.chain = chain;
+        a.y = y;
+        a.chain_bias = bias;
+        a.splits = shape.splits;
+    }
+    const std::uint32_t blocks = shape.groups * shape.splits;
+    hipError_t err = hipErrorInvalidValue;
+    switch (p.type) {
+    case kQ8_0: err = launch_fmt<kQ8_0>(a, shape, blocks, stream); break;
+    case kQ4_0: err = launch_fmt<kQ4_0>(a, shape, blocks, stream); break;
+    case kQ4_K: err = launch_fmt<kQ4_K>(a, shape, blocks, stream); break;
+    default: break;
+    }
+    if (err != hipSuccess || !split || chained) return err;
+    if (epilogue) return launch_split_epilogue(partials, shape.splits, m, p.n, bias, *epilogue, stream);
+    return launch_split_reduce(partials, shape.splits, m, p.n, bias, y, stream);
+}
+
+} // namespace air_hip

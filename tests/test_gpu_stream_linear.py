@@ -1,0 +1,100 @@
+"""The streaming decode linear (linear_stream.hip) on the automatic route.
+
+Shapes at the edges of its tiles: K an odd number of 64-k steps, a tail
+shorter than its chunks, K splits with a short last one, N not a multiple of
+16 and of a workgroup's row tiles, every count of activation tiles; wide
+matrices of one and two tiles per wave.  Each result is held to the oracle at
+relative L2 1e-4 per row, repeats to the same bits, and the no-allocation
+entry point to the same bits too.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from air_amd import capi
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+
+DECODE_TOL = 1e-4
+
+# (format, K, N, widths)
+CASES = [
+    (capi.TYPE_Q8_0, 2080, 5000, (17, 33, 64)),       # 33 steps, 313 row tiles, K splits
+    (capi.TYPE_Q8_0, 4640, 1613, (25, 48)),            # 73 steps, long K, ragged N
+    (capi.TYPE_Q8_0, 2048, 16500, (2, 16, 40)),       # wide, eight tiles a workgroup
+    (capi.TYPE_Q8_0, 2112, 34000, (3, 64)),           # ten
+    (capi.TYPE_Q8_0, 2048, 41000, (9, 33, 49)),       # twenty, two per wave
+    (capi.TYPE_Q4_0, 2144, 4200, (17, 64)),
+    (capi.TYPE_Q4_0, 5152, 1530, (18, 33)),
+    (capi.TYPE_Q4_0, 2048, 41000, (5, 32, 50)),
+    (capi.TYPE_Q4_K, 2304, 4200, (20, 48)),
+    (capi.TYPE_Q4_K, 8448, 1530, (2, 16, 17, 64)),
+    (capi.TYPE_Q4_K, 2048, 41000, (7, 30, 64)),
+]
+
+
+@pytest.mark.parametrize("type_id,k,n,ms", CASES, ids=[f"{capi.TYPE_NAMES[c[0]]}-{c[2]}x{c[1]}" for c in CASES])
+def test_stream_linear(torch_cuda, hip_ctx, type_id, k, n, ms):
+    torch = torch_cuda
+    dev = torch.device("cuda:0")
+    canon = helpers.weights(type_id, k, n, seed=k + n)
+    mat = capi.Matrix(hip_ctx, type_id, k, n, canon, canon.nbytes, on_device=False)
+    rows = np.unique(np.concatenate([np.arange(0, n, max(1, n // 200)), np.arange(max(0, n - 40), n)])).astype(np.uint64)
+    bias = (np.random.default_rng(n).standard_normal(n) * 0.02).astype(np.float32)
+    bias_d = torch.from_numpy(bias).to(dev)
+    try:
+        for m in ms:
+            plan = mat.plan(m)
+            print(f"stream {capi.TYPE_NAMES[type_id]} {n}x{k} M={m}: {plan}", flush=True)
+            assert "stream_kernel" in plan, plan
+            x = helpers.activations(m, k, seed=m + k)
+            x[:, ::61] *= 40.0
+            x[m // 2] *= 1e-5
+            xd = torch.from_numpy(x).to(dev)
+            outs = []
+            for _ in range(2):
+                y = torch.full((m, n), float("nan"), dtype=torch.float32, device=dev)
+                mat.linear(xd, y, m, bias=bias_d)
+                torch.cuda.synchronize()
+                outs.append(y.cpu().numpy())
+            assert np.isfinite(outs[0]).all(), (m, plan)
+            y = torch.full((m, n), float("nan"), dtype=torch.float32, device=dev)
+            mat.linear_noalloc(xd, y, m, bias=bias_d)
+            torch.cuda.synchronize()
+            outs.append(y.cpu().numpy())
+            for other in outs[1:]:
+                assert np.array_equal(outs[0].view(np.uint32), other.view(np.uint32)), (m, plan)
+            want = oracle.linear_row_list(type_id, canon, k, n, x, rows, bias=bias)
+            got = outs[0][:, rows.astype(np.int64)]
+            for r in range(m):
+                assert helpers.rel_l2(got[r], want[r]) <= DECODE_TOL, (m, r, plan)
+    finally:
+        mat.release()
+
+
+def test_stream_outliers_keep_small_channels(torch_cuda, hip_ctx):
+    """A few channels 1e4 times the rest: the error against the small channels'
+    own share of the output stays at 1e-3 (f32 rounding of the outputs)."""
+    torch = torch_cuda
+    k, n, m = 2048, 16500, 24
+    canon = helpers.weights(capi.TYPE_Q4_0, k, n, seed=5)
+    mat = capi.Matrix(hip_ctx, capi.TYPE_Q4_0, k, n, canon, canon.nbytes, on_device=False)
+    try:
+        assert "stream_kernel" in mat.plan(m), mat.plan(m)
+        x = helpers.activations(m, k, seed=6)
+        channels = np.array([3, 700, 1999])
+        x[:, channels] *= np.float32(1e4)
+        small = x.copy()
+        small[:, channels] = 0.0
+        rows = np.arange(0, n, 37).astype(np.uint64)
+        y = torch.empty((m, n), dtype=torch.float32, device="cuda:0")
+        mat.linear(torch.from_numpy(x).to("cuda:0"), y, m)
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()[:, rows.astype(np.int64)].astype(np.float64)
+        want = oracle.linear_row_list(capi.TYPE_Q4_0, canon, k, n, x, rows).astype(np.float64)
+        share = oracle.linear_row_list(capi.TYPE_Q4_0, canon, k, n, small, rows).astype(np.float64)
+        for r in range(m):
+            assert np.linalg.norm(got[r] - want[r]) <= 1e-3 * np.linalg.norm(share[r]), r
+    finally:
+        mat.release()
