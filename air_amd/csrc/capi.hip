@@ -95,6 +95,9 @@ struct air_hip_context {
     void* argmax_partials{nullptr};         // per-slice partials of the greedy selection
     std::uint64_t argmax_partials_bytes{0};
     std::uint64_t attention_scratch_bytes{0};
+    // Split activations of a streaming linear whose rows no epilogue split.
+    void* stream_rows{nullptr};
+    std::uint64_t stream_rows_bytes{0};
     void* epilogue_rows{nullptr};           // linear output of air_hip_linear_epilogue's unfused route
     std::uint64_t epilogue_rows_bytes{0};
     // This device's `scratch` array (hipGetSymbolAddress at context creation).
@@ -321,7 +324,8 @@ int run_prefill(air_hip_context* ctx, const air_hip_matrix* m, const float* x, f
 }
 
 int ensure_split_buffers(air_hip_context* ctx, std::uint64_t partial_bytes, std::uint32_t counters);
-std::uint64_t* chain_for(air_hip_context* ctx, std::uint32_t splits, std::uint32_t m, std::uint64_t n);
+std::uint64_t* chain_for(air_hip_context* ctx, std::uint32_t splits, std::uint32_t m, std::uint64_t n,
+                         bool stream = false);
 int linear_loaded(air_hip_context* ctx, const air_hip_matrix* m, float* y, const float* bias, int tactic,
                   const SplitEpilogue* epilogue, bool* applied);
 
@@ -365,6 +369,23 @@ bool decode_automatic(const air_hip_context* ctx) {
 SkinnyShape skinny_plan(const air_hip_context* ctx, const TilePlanes& p, std::uint32_t rows) {
     if (decode_automatic(ctx) && stream_preferred(p, rows)) return plan_stream(p, rows);
     return plan_skinny(p, rows, ctx->skinny_tile_n, ctx->skinny_splits, ctx->skinny_lds_stages, ctx->skinny_waves);
+}
+
+// A dense F16 or Q6_K matrix at decode widths runs the streaming kernel on
+// its rows where the automatic route prefers it and what it needs fits the
+// no-allocation entry point's scratch (so both entry points take one route).
+bool dense_stream(const air_hip_context* ctx, const air_hip_matrix* m, std::uint32_t rows, int tactic) {
+    const DenseTuning& t = ctx->dense_tuning;
+    if (!m->dense || !m->gemm.codes || tactic == AIR_HIP_LINEAR_PREFILL || rows > AIR_HIP_MAX_DECODE_ROWS ||
+        t.path != 0u || t.shape.tile_n != 0u || t.shape.waves != 0u || t.shape.depth != 0u ||
+        (m->dense_storage != kF16 && m->dense_storage != kQ6_K) || !decode_automatic(ctx) ||
+        !stream_preferred(m->gemm, rows)) {
+        return false;
+    }
+    const SkinnyShape s = plan_stream(m->gemm, rows);
+    const std::uint64_t kp = ceil_div(m->gemm.k, kSplitK) * kSplitK;
+    return ceil_div(split_workspace_bytes(kp, rows), 256u) * 256u + skinny_partials_bytes(s, rows, m->gemm.n) <=
+           kNoAllocScratchBytes;
 }
 
 // The skinny kernel straight from the f32 rows, or over activations split
@@ -416,11 +437,46 @@ Route route_linear(const air_hip_context* ctx, const air_hip_matrix* m, std::uin
     return Route::decode_linear;
 }
 
+// The streaming decode linear over `planes` (the matrix's tiles or dense
+// rows).  Its activations are the split an epilogue just left for these rows
+// (`ready`), or are split into a buffer of its own: activations a caller
+// loaded stay as they are.
+int run_stream(air_hip_context* ctx, const air_hip_matrix* m, const TilePlanes& planes, const float* x, float* y,
+               const float* bias, std::uint32_t rows, const SplitEpilogue* epilogue, bool* applied, const void* ready) {
+    const SkinnyShape shape = plan_stream(planes, rows);
+    const std::uint64_t kp = ceil_div(planes.k, kSplitK) * kSplitK;
+    SplitWorkspace ws{};
+    if (ready == x && ctx->loaded_k == planes.k && ctx->loaded_rows == rows && ctx->loaded_row_scaled) {
+        ws = carve_split_workspace(ctx->workspace, kp, rows);
+    } else {
+        const int rc = grow_buffer(ctx, &ctx->stream_rows, &ctx->stream_rows_bytes, split_workspace_bytes(kp, rows),
+                                   "stream activations");
+        if (rc != AIR_HIP_OK) return rc;
+        ws = carve_split_workspace(ctx->stream_rows, kp, rows);
+        const hipError_t err = launch_split_activations_rows(x, rows, planes.k, kp, ws, ctx->stream);
+        if (err != hipSuccess) return hip_fail(err, "split_rows_kernel");
+    }
+    const std::uint64_t partial_bytes = skinny_partials_bytes(shape, rows, planes.n);
+    if (partial_bytes > 0u) {
+        const int rc = ensure_split_buffers(ctx, partial_bytes, 0u);
+        if (rc != AIR_HIP_OK) return rc;
+    }
+    const SplitEpilogue* epi = reduction_epilogue(ctx, m, shape, bias, rows, epilogue, applied);
+    std::uint64_t* chain = epi ? nullptr : chain_for(ctx, shape.splits, rows, planes.n, true);
+    const hipError_t err = launch_stream_linear(planes, ws, bias, y, rows, shape,
+                                                static_cast<float*>(ctx->split_partials), ctx->stream, epi, chain);
+    if (err != hipSuccess) return hip_fail(err, "stream_kernel");
+    ctx->decode_linear_calls.fetch_add(1, std::memory_order_relaxed);
+    ctx->decode_rows.fetch_add(rows, std::memory_order_relaxed);
+    return AIR_HIP_OK;
+}
+
 // Skinny decode linear straight from the f32 rows (M = 2..64): one launch
 // (two with a K split), no activation workspace.
 int run_skinny_x(air_hip_context* ctx, const air_hip_matrix* m, const float* x, float* y, const float* bias,
                  std::uint32_t rows, const SplitEpilogue* epilogue, bool* applied, const void* ready) {
     const SkinnyShape shape = skinny_plan(ctx, m->planes, rows);
+    if (shape.stream) return run_stream(ctx, m, m->planes, x, y, bias, rows, epilogue, applied, ready);
     if (skinny_route(ctx, m, rows) == Route::skinny_loaded) {
         int rc = load_activations_for(ctx, x, m->planes.k, rows, ready);
         if (rc != AIR_HIP_OK) return rc;
@@ -482,17 +538,21 @@ int run_wsplit(air_hip_context* ctx, const air_hip_matrix* m, const float* x, fl
 // further split adds a level of exchanges that an output passes in turn, so
 // 8-way splits gain only at about 50k outputs (down at 2 rows) and lose 3-42
 // us beyond.
-bool chain_auto(std::uint32_t splits, std::uint32_t m, std::uint64_t n) {
+// The streaming kernel takes only two-way splits that way: its splits end
+// together, and a longer chain is walked level by level (Q6_K down at 2 rows,
+// nine splits: 34.4 us against 33.1 for 5 rows with the reduction).
+bool chain_auto(std::uint32_t splits, std::uint32_t m, std::uint64_t n, bool stream) {
     const std::uint64_t outputs = static_cast<std::uint64_t>(m) * n;
+    if (stream && splits > 2u) return false;
     return (splits == 2u && outputs <= (256u << 10)) || outputs * (splits - 1u) <= (56u << 10);
 }
 
 // The chain slots for a K split of `splits` over m x n outputs, or null for
 // the reduction launch: the mode asks for it, or the slots would have to grow
 // (and be zeroed) while the stream is being captured.
-std::uint64_t* chain_for(air_hip_context* ctx, std::uint32_t splits, std::uint32_t m, std::uint64_t n) {
+std::uint64_t* chain_for(air_hip_context* ctx, std::uint32_t splits, std::uint32_t m, std::uint64_t n, bool stream) {
     if (splits < 2u || ctx->chain_mode == 1u) return nullptr;
-    if (ctx->chain_mode == 0u && !chain_auto(splits, m, n)) return nullptr;
+    if (ctx->chain_mode == 0u && !chain_auto(splits, m, n, stream)) return nullptr;
     const std::uint64_t bytes = chain_slot_bytes(splits, m, n);
     if (bytes <= ctx->chain_slots_bytes) return ctx->chain_slots;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
@@ -736,6 +796,7 @@ int air_hip_context_destroy(air_hip_context* ctx) {
         if (ctx->attention_scratch) (void)hipFree(ctx->attention_scratch);
         if (ctx->argmax_partials) (void)hipFree(ctx->argmax_partials);
         if (ctx->epilogue_rows) (void)hipFree(ctx->epilogue_rows);
+        if (ctx->stream_rows) (void)hipFree(ctx->stream_rows);
         if (ctx->gemv_pairs) (void)hipFree(ctx->gemv_pairs);
         if (ctx->chain_slots) (void)hipFree(ctx->chain_slots);
         for (void* p : ctx->retired) (void)hipFree(p);
@@ -757,6 +818,11 @@ int air_hip_context_reserve(air_hip_context* ctx, uint64_t max_k, uint32_t max_m
     if (scope.status() != hipSuccess) return hip_fail(scope.status(), "hipSetDevice");
     const std::uint64_t kp = ceil_div(max_k, kSplitK) * kSplitK;
     int rc = ensure_workspace(ctx, split_workspace_bytes(kp, max_m < kMaxRows ? max_m : kMaxRows));
+    if (rc == AIR_HIP_OK && max_m > 1u) {
+        rc = grow_buffer(ctx, &ctx->stream_rows, &ctx->stream_rows_bytes,
+                         split_workspace_bytes(kp, std::min<std::uint32_t>(max_m, AIR_HIP_MAX_DECODE_ROWS)),
+                         "stream activations");
+    }
     if (rc != AIR_HIP_OK || max_m <= kFusedMaxRows) return rc;
     PrefillShape unsplit{};
     return ensure_prefill_workspace(ctx, prefill_workspace_bytes(max_k, max_m < kMaxRows ? max_m : kMaxRows, unsplit, 0));
@@ -1197,7 +1263,7 @@ int linear_loaded(air_hip_context* ctx, const air_hip_matrix* m, float* y, const
             if (rc != AIR_HIP_OK) return rc;
         }
         const SplitEpilogue* epi = reduction_epilogue(ctx, m, shape, bias, rows, epilogue, applied);
-        std::uint64_t* chain = epi ? nullptr : chain_for(ctx, shape.splits, rows, m->planes.n);
+        std::uint64_t* chain = epi ? nullptr : chain_for(ctx, shape.splits, rows, m->planes.n, shape.stream);
         const hipError_t err = launch_skinny_linear(m->planes, ws, bias, y, rows, shape,
                                                     static_cast<float*>(ctx->split_partials), ctx->stream, epi, chain);
         if (err != hipSuccess) return hip_fail(err, "skinny_kernel");
@@ -1237,6 +1303,7 @@ int linear_rows(air_hip_context* ctx, const air_hip_matrix* m, const float* x, f
             return run_prefill(ctx, m, x, y, bias, rows, prefill_ready, ctx->prefill_source_k, ctx->prefill_source_rows,
                                epilogue, applied);
         }
+        if (dense_stream(ctx, m, rows, tactic)) return run_stream(ctx, m, m->gemm, x, y, bias, rows, epilogue, applied, ready);
         const hipError_t err = launch_dense_linear(m->dense, m->dense_storage, m->planes.k, m->planes.n, x, bias, y, rows,
                                                      ctx->stream, ctx->dense_tuning);
         if (err != hipSuccess) return hip_fail(err, "dense_rows_kernel / dense_gemm_kernel");
@@ -1289,9 +1356,10 @@ int linear_rows(air_hip_context* ctx, const air_hip_matrix* m, const float* x, f
 }
 
 // How a plain linear's K split of `splits` workgroups is summed.
-const char* split_tail(const air_hip_context* ctx, std::uint32_t splits, std::uint32_t m, std::uint64_t n) {
+const char* split_tail(const air_hip_context* ctx, std::uint32_t splits, std::uint32_t m, std::uint64_t n,
+                       bool stream = false) {
     if (splits < 2u) return "";
-    const bool chain = ctx->chain_mode == 2u || (ctx->chain_mode == 0u && chain_auto(splits, m, n));
+    const bool chain = ctx->chain_mode == 2u || (ctx->chain_mode == 0u && chain_auto(splits, m, n, stream));
     return chain ? " + in-kernel chain" : " + split reduction";
 }
 
@@ -1320,6 +1388,14 @@ std::string describe_linear(const air_hip_context* ctx, const air_hip_matrix* m,
             const Q6kGemvPlan g = plan_q6k_gemv(m->planes.k, m->planes.n, ctx->dense_tuning.shape);
             std::snprintf(buf, sizeof buf, "q6k_gemv_kernel waves=%u units=%u depth=%u (dense q6_k super-block rows)",
                           g.waves, g.units, g.depth);
+            break;
+        }
+        if (dense_stream(ctx, m, rows, tactic)) {
+            const SkinnyShape k = plan_stream(m->gemm, rows);
+            std::snprintf(buf, sizeof buf, "split_rows_kernel + stream_kernel<%s> mt=%u tile_n=%u waves=%u+2 groups=%u "
+                          "splits=%u%s (dense %s %s)", t, k.mt, k.tile_n, k.waves, k.groups, k.splits,
+                          split_tail(ctx, k.splits, rows, m->planes.n, true), t,
+                          m->type == kQ6_K ? "super-block rows" : "rows");
             break;
         }
         if (dense_mfma_route(m->dense_storage, m->planes.k, m->planes.n, rows, ctx->dense_tuning)) {
@@ -1375,7 +1451,7 @@ std::string describe_linear(const air_hip_context* ctx, const air_hip_matrix* m,
         if (k.stream) {
             std::snprintf(buf, sizeof buf, "split_rows_kernel + stream_kernel<%s> mt=%u tile_n=%u waves=%u+2 groups=%u "
                           "splits=%u%s", fmt, k.mt, k.tile_n, k.waves, k.groups, k.splits,
-                          split_tail(ctx, k.splits, rows, m->planes.n));
+                          split_tail(ctx, k.splits, rows, m->planes.n, true));
             break;
         }
         const bool lds = loaded && k.lds_stages >= 2u;
@@ -1429,9 +1505,22 @@ int air_hip_linear_noalloc(air_hip_context* ctx, const air_hip_matrix* m, const 
     }
     if (m->owner->device != ctx->device) return fail(AIR_HIP_INVALID_ARGUMENT, "matrix belongs to another device");
     if (reinterpret_cast<std::uintptr_t>(x) % 16u != 0) return fail(AIR_HIP_INVALID_ARGUMENT, "x must be 16-byte aligned");
-    if (m->dense) {   // no scratch: the same launch as air_hip_linear
+    if (m->dense) {   // the same launches as air_hip_linear
         DeviceScope scope(ctx->device);
         if (scope.status() != hipSuccess) return hip_fail(scope.status(), "hipSetDevice");
+        if (ctx->noalloc_scratch && dense_stream(ctx, m, rows, tactic)) {
+            const SkinnyShape shape = plan_stream(m->gemm, rows);
+            const std::uint64_t kp = ceil_div(m->gemm.k, kSplitK) * kSplitK;
+            auto* base = static_cast<unsigned char*>(ctx->noalloc_scratch);
+            const SplitWorkspace ws = carve_split_workspace(base, kp, rows);
+            float* partials = reinterpret_cast<float*>(base + ceil_div(split_workspace_bytes(kp, rows), 256u) * 256u);
+            hipError_t err = launch_split_activations_rows(x, rows, m->gemm.k, kp, ws, ctx->stream);
+            if (err == hipSuccess) err = launch_stream_linear(m->gemm, ws, bias, y, rows, shape, partials, ctx->stream);
+            if (err != hipSuccess) return hip_fail(err, "stream_kernel");
+            ctx->decode_linear_calls.fetch_add(1, std::memory_order_relaxed);
+            ctx->decode_rows.fetch_add(rows, std::memory_order_relaxed);
+            return AIR_HIP_OK;
+        }
         const hipError_t err = launch_dense_linear(m->dense, m->dense_storage, m->planes.k, m->planes.n, x, bias, y, rows,
                                                      ctx->stream, ctx->dense_tuning);
         if (err != hipSuccess) return hip_fail(err, "dense_rows_kernel / dense_gemm_kernel");

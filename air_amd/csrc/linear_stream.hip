@@ -1,5 +1,5 @@
 // linear_stream.hip -- the decode linear for M = 2..64 rows over split
-// activations: weights streamed through registers, activations shared through
+// activations, in the tile formats and over dense F16 and Q6_K rows: weights streamed through registers, activations shared through
 // LDS by waves that do nothing else.
 //
 // The arithmetic of skinny_kernel / skinny_lds_kernel (linear_skinny.hip);
@@ -48,6 +48,12 @@
 //           Q4_0  91 -> 73        92 -> 78      126 -> 107    197 -> 169
 //           Q4_K  115 -> 89       112 -> 90     158 -> 130    253 -> 206
 //
+// Dense rows (dense_mfma_kernel before, which asks for a Q6_K step in eight
+// 4-byte loads a lane; here a super-block is three 16-byte loads and its
+// scales): Q6_K down at 13 rows 63.8 -> 34.0, at 64 201 -> 60.4; gate|up 93.6
+// -> 43.2 and 255 -> 89.1; lm_head 331 -> 136 and 948 -> 327; F16 gate|up at 24
+// rows 99 -> 78.7, at 64 286 -> 90.3; down at 64 154 -> 62.9.
+//
 // Replaces specialized_matmul_kernel / specialized_matmul_batch_reuse_kernel
 // (src/cuda/cuda_backend.cu:501-583) for batched decode.
 #include "air_hip_device.hpp"
@@ -61,11 +67,13 @@
 namespace air_hip {
 namespace {
 
+typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+
 struct StreamArgs {
-    const void* codes;
-    const void* scales;
+    const void* codes;           // tile codes, or dense rows (F16) / records (Q6_K)
+    const void* scales;          // tile scales, or the records' f16 d plane (Q6_K)
     std::uint32_t nt, kt;
-    std::uint64_t n;
+    std::uint64_t n, k;
     const u32x4* xs;             // split activations [block][MT][2][64] x 16 B
     std::uint32_t blocks;        // 32-element blocks of the workspace
     const float* inv_scale;      // [mp] inverse power-of-two scale of each row
@@ -133,8 +141,63 @@ struct Record<kQ4_K> {
     u32x4 h;
 };
 
+// Dense storage: F16 rows as they are (both blocks of a step), Q6_K
+// super-blocks as linear_dense.hip records (a lane group's 48 code bytes, the
+// row's sixteen sub-block scales, d).
+template <>
+struct Record<kF16> {
+    u32x4 v[2];
+};
+template <>
+struct Record<kQ6_K> {
+    u32x4 c[3];
+    u32x4 s;
+    std::uint32_t d;
+};
+
 template <int FMT>
-constexpr unsigned kUnit = FMT == kQ8_0 ? 1u : FMT == kQ4_0 ? 2u : 4u;   // 64-k steps per record
+constexpr unsigned kUnit = FMT == kQ8_0 || FMT == kF16 ? 1u : FMT == kQ4_0 ? 2u : 4u;   // 64-k steps per record
+
+constexpr unsigned kQ6kRecord = 208u;
+
+// Record `unit` of the lane's row of a dense matrix.
+template <int FMT>
+__device__ __forceinline__ void load_dense_record(const StreamArgs& a, std::uint64_t row, std::uint32_t unit,
+                                                  std::uint32_t lane, Record<FMT>& out) {
+    const unsigned char* base = static_cast<const unsigned char*>(a.codes);
+    const std::uint32_t g = lane >> 4;
+    if constexpr (FMT == kQ6_K) {
+        const std::uint64_t blk = row * (a.k / 256u) + unit;
+        const unsigned char* rec = base + blk * kQ6kRecord;
+#pragma unroll
+        for (unsigned i = 0; i < 3u; ++i) {
+            out.c[i] = *reinterpret_cast<const u32x4*>(rec + q6k_code_offset(g, 16u * i));
+        }
+        out.s = *reinterpret_cast<const u32x4*>(rec + 192u);
+        out.d = static_cast<const std::uint16_t*>(a.scales)[blk];
+    } else {
+        // A row that ends on the first block of a step has no second one.
+        const std::uint64_t col = static_cast<std::uint64_t>(unit) * kStepK + 8u * g;
+        const unsigned char* at = base + (row * a.k + col) * 2u;
+        const bool both = col + 32u < a.k;
+        out.v[0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(at));
+        out.v[1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(at + (both ? 64u : 0u)));
+        if (!both) out.v[1] = u32x4{0u, 0u, 0u, 0u};
+    }
+}
+
+// Four 6-bit codes (low nibbles `nibble` of ql's bytes, high pairs at bits
+// `pair` of qh's) as exact f16 values q - 32.
+template <unsigned nibble, unsigned pair>
+__device__ __forceinline__ half4v q6_codes(std::uint32_t ql, std::uint32_t qh) {
+    const std::uint32_t low = (ql >> (4u * nibble)) & 0x0f0f0f0fu;
+    const std::uint32_t high = (pair < 4u ? qh << (4u - pair) : qh >> (pair - 4u)) & 0x30303030u;
+    const std::uint32_t q = low | high;
+    const half2v bias = {(_Float16)1056.0f, (_Float16)1056.0f};
+    const half2v p0 = bits_as_half2(__builtin_amdgcn_perm(0x64646464u, q, 0x04010400u)) - bias;
+    const half2v p1 = bits_as_half2(__builtin_amdgcn_perm(0x64646464u, q, 0x04030402u)) - bias;
+    return half4v{p0[0], p0[1], p1[0], p1[1]};
+}
 
 template <int FMT>
 __device__ __forceinline__ void load_record(const void* codes, const void* scales, std::uint64_t tile,
@@ -179,13 +242,16 @@ constexpr unsigned kBuffers = 4u;
 // Weight records in flight per wave: 8 KiB of codes (Q8_0), less where three
 // or four activation tiles need the registers.
 template <int FMT, int MT, int TN>
-constexpr unsigned kRing = FMT == kQ8_0   ? (MT <= 2 ? 8u : 4u) / TN
+constexpr unsigned kRing = FMT == kQ8_0 || FMT == kF16 ? (MT <= 2 ? 8u : 4u) / TN
                            : FMT == kQ4_0 ? (MT <= 2 && TN == 1 ? 4u : 2u)
-                                          : (TN == 1 ? 2u : 1u);
+                                          : (TN == 1 && (FMT == kQ4_K || MT <= 2) ? 2u : 1u);   // Q4_K, Q6_K
 constexpr int kProducers = 2;
 // Levels of the K sum: three, or as many as leave no register in scratch.
 template <int FMT, int MT, int TN>
-constexpr unsigned kLevels = MT <= 2 ? 3u : FMT == kQ4_K || (MT == 4 && TN == 2) ? 1u : 2u;
+constexpr unsigned kLevels = FMT == kF16 && MT == 2 && TN == 2 ? 2u
+                             : MT <= 2 || FMT == kQ6_K         ? 3u
+                             : FMT == kQ4_K || (MT == 4 && TN == 2) ? 1u
+                                                                    : 2u;
 
 template <int FMT, int MT, int TN, int W>
 __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) void stream_kernel(StreamArgs a) {
@@ -193,10 +259,16 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
     constexpr unsigned U = kUnit<FMT>;
     constexpr unsigned D = kRing<FMT, MT, TN>;
     constexpr unsigned C = kChunk<MT>;
-    constexpr unsigned kBody = D * U > C ? D * U : C;       // steps per trip: the ring comes full circle
-    constexpr bool kSums = FMT == kQ4_K;
-    constexpr unsigned kMp = 16u * MT;
     constexpr unsigned L = kLevels<FMT, MT, TN>;
+    // Steps per trip: the ring comes full circle.  At three levels the second
+    // one covers eight steps (two trips of four with four activation tiles,
+    // which would spill in a trip of eight).
+    constexpr bool kEight = L > 2u && MT <= 3;
+    constexpr unsigned kBody = D * U > C && D * U > (kEight ? 8u : 0u) ? D * U : kEight && C < 8u ? 8u : C;
+    constexpr bool kHold = L > 2u && kBody < 8u;
+    constexpr bool kSums = FMT == kQ4_K;
+    constexpr bool kDense = dense_storage(FMT);
+    constexpr unsigned kMp = 16u * MT;
     constexpr unsigned kParts = MT <= 2 ? 2u : 1u;
     constexpr unsigned kFrags = 2u * C * 2u * MT;           // 1 KiB activation fragments per chunk
     constexpr unsigned kXBytes = kFrags * 1024u;
@@ -262,13 +334,20 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
     std::uint64_t wtile[TN];
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-        wtile[j] = static_cast<std::uint64_t>(min(rt0 + static_cast<std::uint32_t>(j), a.nt - 1u)) * a.kt;
+        if constexpr (kDense) {   // the lane's row
+            wtile[j] = min(static_cast<std::uint64_t>(rt0 + static_cast<std::uint32_t>(j)) * 16u + (lane & 15u), a.n - 1u);
+        } else {
+            wtile[j] = static_cast<std::uint64_t>(min(rt0 + static_cast<std::uint32_t>(j), a.nt - 1u)) * a.kt;
+        }
     }
     Record<FMT> ring[D][TN];
     const auto load_w = [&](Record<FMT>(&dst)[TN], std::uint32_t unit) __attribute__((always_inline)) {
         const std::uint32_t u = min(unit, u_last);
 #pragma unroll
-        for (int j = 0; j < TN; ++j) load_record<FMT>(a.codes, a.scales, wtile[j] + u, lane, dst[j]);
+        for (int j = 0; j < TN; ++j) {
+            if constexpr (kDense) load_dense_record<FMT>(a, wtile[j], u, lane, dst[j]);
+            else load_record<FMT>(a.codes, a.scales, wtile[j] + u, lane, dst[j]);
+        }
     };
     // Stage q of a chunk (compile time): its fragments from LDS, read one
     // stage ahead of the arithmetic so that no MFMA waits for an LDS read.  A
@@ -283,7 +362,15 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
 #pragma unroll
             for (unsigned i = 0; i < kParts; ++i) {
                 const unsigned f = (blk * MT + static_cast<unsigned>(t)) * 2u + (kParts == 2u ? i : q % 2u);
-                frag[q & 1u][t][i] = *reinterpret_cast<const half8v*>(base + f * 1024u + lane * 16u);
+                if constexpr (FMT == kQ6_K) {
+                    // Elements 4 (l / 16)..+3 of both 16-element halves, as
+                    // its 16-weight sub-blocks take them.
+                    const unsigned char* at = base + f * 1024u + ((lane & 15u) + 16u * (lane >> 5)) * 16u + 8u * ((lane >> 4) & 1u);
+                    const u32x2 h0 = *reinterpret_cast<const u32x2*>(at), h1 = *reinterpret_cast<const u32x2*>(at + 512u);
+                    frag[q & 1u][t][i] = __builtin_bit_cast(half8v, u32x4{h0.x, h0.y, h1.x, h1.y});
+                } else {
+                    frag[q & 1u][t][i] = *reinterpret_cast<const half8v*>(base + f * 1024u + lane * 16u);
+                }
             }
         }
     };
@@ -295,7 +382,9 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
         constexpr unsigned q = blk * 2u / kParts;       // the block's first stage
         half8v w[TN];
         float ws[TN], wo[TN];
+        float ws2[FMT == kQ6_K ? TN : 1];               // the block's second sub-block
         float4v p[TN][MT];
+        float4v p2[FMT == kQ6_K ? TN : 1][FMT == kQ6_K ? MT : 1];
         if constexpr (!LAST || kParts == 1u) read_stage.template operator()<q + 1u>(base);
         const auto read_sums = [&]() __attribute__((always_inline)) {
             if constexpr (kSums) {
@@ -310,14 +399,51 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            const StepCodes<FMT> w_step = record_step<FMT, sub>(w_in[j]);
-            w[j] = step_codes<FMT>(w_step, b);
-            step_scale<FMT>(w_step, sub, b, ws[j], wo[j]);
+            if constexpr (FMT == kF16) {
+                w[j] = __builtin_bit_cast(half8v, w_in[j].v[b]);
+            } else if constexpr (FMT == kQ6_K) {
+                // Half `sub / 2`, quadrant 2 (sub % 2) + b: dwords {low
+                // nibbles of even, odd quadrants, high pairs} per
+                // half-quadrant (linear_dense.hip).
+                constexpr unsigned d0 = 6u * (sub >> 1), d1 = d0 + 3u, pair = 4u * (sub & 1u) + 2u * b;
+                const auto word = [&](unsigned i) { return w_in[j].c[i / 4u][i % 4u]; };
+                const half4v c0 = q6_codes<sub & 1u, pair>(word(d0 + b), word(d0 + 2u));
+                const half4v c1 = q6_codes<sub & 1u, pair>(word(d1 + b), word(d1 + 2u));
+                w[j] = __builtin_shufflevector(c0, c1, 0, 1, 2, 3, 4, 5, 6, 7);
+                const float d = f16_bits_value(w_in[j].d);
+                const int sc = static_cast<int>(w_in[j].s[sub]);
+                ws[j] = d * static_cast<float>((sc << (24u - 16u * b)) >> 24);
+                ws2[j] = d * static_cast<float>((sc << (16u - 16u * b)) >> 24);
+            } else {
+                const StepCodes<FMT> w_step = record_step<FMT, sub>(w_in[j]);
+                w[j] = step_codes<FMT>(w_step, b);
+                step_scale<FMT>(w_step, sub, b, ws[j], wo[j]);
+            }
         }
+        const auto lower = [](const half8v& v) { return __builtin_shufflevector(v, v, 0, 1, 2, 3); };
+        const auto upper = [](const half8v& v) { return __builtin_shufflevector(v, v, 4, 5, 6, 7); };
+        // First products of a block, then the low parts on top of them.
+        const auto first = [&](int j, int t, const half8v& f) __attribute__((always_inline)) {
+            const float4v zero{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (FMT == kQ6_K) {
+                p[j][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(lower(f), lower(w[j]), zero, 0, 0, 0);
+                p2[j][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(upper(f), upper(w[j]), zero, 0, 0, 0);
+            } else {
+                p[j][t] = mfma16x16x32(f, w[j], zero);
+            }
+        };
+        const auto second = [&](int j, int t, const half8v& f) __attribute__((always_inline)) {
+            if constexpr (FMT == kQ6_K) {
+                p[j][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(lower(f), lower(w[j]), p[j][t], 0, 0, 0);
+                p2[j][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(upper(f), upper(w[j]), p2[j][t], 0, 0, 0);
+            } else {
+                p[j][t] = mfma16x16x32(f, w[j], p[j][t]);
+            }
+        };
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int t = 0; t < MT; ++t) p[j][t] = mfma16x16x32(frag[q & 1u][t][0], w[j], float4v{0.0f, 0.0f, 0.0f, 0.0f});
+            for (int t = 0; t < MT; ++t) first(j, t, frag[q & 1u][t][0]);
         if constexpr (kParts == 1u) {
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (!LAST) read_stage.template operator()<q + 2u>(base);
@@ -328,15 +454,22 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
-                p[j][t] = mfma16x16x32(kParts == 2u ? frag[q & 1u][t][kParts - 1u] : frag[(q + 1u) & 1u][t][0], w[j], p[j][t]);
+                second(j, t, kParts == 2u ? frag[q & 1u][t][kParts - 1u] : frag[(q + 1u) & 1u][t][0]);
             }
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
                 float4v& sum = L > 2u ? pair[j][t] : L > 1u ? part[j][t] : acc[j][t];
-                if constexpr (L > 2u && blk % 4u == 0u) sum = ws[j] * p[j][t];
-                else sum += ws[j] * p[j][t];
+                if constexpr (FMT == kF16) {
+                    if constexpr (L > 2u && blk % 4u == 0u) sum = p[j][t];
+                    else sum += p[j][t];
+                } else if constexpr (L > 2u && blk % 4u == 0u) {
+                    sum = ws[j] * p[j][t];
+                } else {
+                    sum += ws[j] * p[j][t];
+                }
+                if constexpr (FMT == kQ6_K) sum += ws2[j] * p2[j][t];
                 if constexpr (kSums) sum -= wo[j] * sums[t];
                 if constexpr (L > 2u && blk % 4u == 3u) part[j][t] += sum;
             }
@@ -349,10 +482,11 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
     });
     // One trip: kBody steps from s.  WHOLE: all of them lie in the range.
     std::uint32_t buffer = 0u;
+    bool first_half = true;   // kHold: of the second level's eight steps
     const auto trip = [&](std::uint32_t s, auto whole_tag) __attribute__((always_inline)) {
         constexpr bool WHOLE = decltype(whole_tag)::value;
         bool done = false;
-        if constexpr (L > 1u) {
+        if (L > 1u && (!kHold || first_half)) {
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -389,12 +523,20 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
                 if constexpr (L > 2u) {
                     if (open) part[j][t] += pair[j][t];
                 }
-                if constexpr (L > 1u) acc[j][t] += part[j][t];
+                if (L > 1u && (!kHold || !first_half || !WHOLE)) acc[j][t] += part[j][t];
             }
+        if constexpr (kHold) first_half = !first_half;
     };
     std::uint32_t s = s_begin;
     for (; s + kBody <= s_end; s += kBody) trip(s, std::true_type{});
-    if (s < s_end) trip(s, std::false_type{});
+    if (s < s_end) {
+        trip(s, std::false_type{});
+    } else if (kHold && !first_half) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[j][t] += part[L > 1u ? j : 0][L > 1u ? t : 0];
+    }
 
     // D[row = activation row][col = weight row], as skinny_kernel.
     float4v inv[MT];
@@ -434,7 +576,9 @@ hipError_t launch_w(const StreamArgs& a, std::uint32_t blocks, hipStream_t strea
 
 template <int FMT, int MT>
 hipError_t launch_mt(const StreamArgs& a, const SkinnyShape& s, std::uint32_t blocks, hipStream_t stream) {
-    if (s.waves == 10u && s.tile_n == 2u) return launch_w<FMT, MT, 2, 10>(a, blocks, stream);
+    if constexpr (!(FMT == kQ6_K && MT >= 3)) {
+        if (s.waves == 10u && s.tile_n == 2u) return launch_w<FMT, MT, 2, 10>(a, blocks, stream);
+    }
     if (s.waves == 10u && s.tile_n == 1u) return launch_w<FMT, MT, 1, 10>(a, blocks, stream);
     if (s.waves == 8u && s.tile_n == 1u) return launch_w<FMT, MT, 1, 8>(a, blocks, stream);
     return hipErrorInvalidConfiguration;
@@ -453,8 +597,8 @@ hipError_t launch_fmt(const StreamArgs& a, const SkinnyShape& s, std::uint32_t b
 } // namespace
 
 bool stream_preferred(const TilePlanes& p, std::uint32_t m) {
-    // Measured against the kernels it replaces on the Qwen2-7B matrices in all
-    // three formats at M = 3, 8, 16, 20, 32, 48 and 64 (graph replay, split
+    // Measured against the kernels it replaces on the Qwen2-7B matrices in the
+    // tile formats at M = 3, 8, 16, 20, 32, 48 and 64 (graph replay, split
     // launch included; the table at the top):
     //  * wide matrices (over 1024 row tiles): faster at every width, but for
     //    Q8_0 ones of 2000..4096 row tiles at 17..32 rows, whose eight-wave
@@ -471,6 +615,21 @@ bool stream_preferred(const TilePlanes& p, std::uint32_t m) {
     // the wave-split kernel, 31.6 here).
     if (m < 2u || m > 64u || p.kp / kStepK < 32u) return false;
     const bool one = m <= 16u, two = !one && m <= 32u;
+    if (p.type == kQ6_K) {
+        // Against dense_mfma_kernel: 1.1 to 3.5 times faster but for narrow
+        // short-K matrices below 16 rows (o at 13 rows 14.7 against 15.2 us).
+        return p.nt >= 96u && (m >= 16u || p.nt > 256u || p.k > 4096u);
+    }
+    if (p.type == kF16) {
+        // Against dense_mfma_kernel, which reads the weights once for 64 rows
+        // too but from half the waves: from 17 rows (gate|up at 24 99 -> 79
+        // us, 13 even; down 79 -> 59), later on narrow (o at 48 rows 28.5
+        // against 29.2) and short-K ones (688 tiles of K = 2048 at 24 rows
+        // 28.6 against 30.0, at 48 46 -> 33).
+        if (m <= 16u || p.nt < 96u) return false;
+        if (two) return p.nt > 1024u || (p.nt > 256u && p.k >= 3072u) || p.k > 8192u;
+        return p.nt > 256u || p.k > 4096u || m > 48u;
+    }
     if (p.nt > 1024u) return !(p.type == kQ8_0 && two && p.nt >= 2000u && p.nt <= 4096u);
     if (p.nt < 96u) return false;
     const bool long_k = p.k > 4096u;
@@ -489,7 +648,7 @@ SkinnyShape plan_stream(const TilePlanes& p, std::uint32_t m) {
     // workgroup, ten from 2049 row tiles, twenty (two per wave, which also
     // halves the activations read per tile: lm_head 141 -> 121 us at 32 rows)
     // from 2561, where ten would start a second round.
-    s.tile_n = p.nt > 2560u ? 2u : 1u;
+    s.tile_n = p.nt > 2560u && !(p.type == kQ6_K && s.mt >= 3u) ? 2u : 1u;   // (that one would spill)
     s.waves = p.nt > 2048u ? 10u : 8u;
     s.groups = static_cast<std::uint32_t>(ceil_div(p.nt, s.waves * s.tile_n));
     // Otherwise K is split over workgroups up to that round, at least twelve
@@ -497,11 +656,11 @@ SkinnyShape plan_stream(const TilePlanes& p, std::uint32_t m) {
     // four splits, 17.6 with seven; ten with three or four activation tiles
     // and eight for Q4_K, whose steps take longer: 18.4 and 17.3 us with four
     // and six), and no further than plan_skinny would.
-    const std::uint32_t least = p.type == kQ4_K ? 8u : s.mt >= 3u ? 10u : 12u;
+    const std::uint32_t least = p.type == kQ4_K || p.type == kQ6_K ? 8u : s.mt >= 3u ? 10u : 12u;
     std::uint32_t splits = std::min(256u / std::min(s.groups, 256u), s.steps / least);
-    splits = std::min(splits, plan_skinny(p, m, 0u, 0u).splits);
+    if (!dense_storage(p.type)) splits = std::min(splits, plan_skinny(p, m, 0u, 0u).splits);
     splits = std::max(splits, 1u);
-    const std::uint32_t unit = p.type == kQ8_0 ? kUnit<kQ8_0> : p.type == kQ4_0 ? kUnit<kQ4_0> : kUnit<kQ4_K>;
+    const std::uint32_t unit = p.type == kQ8_0 || p.type == kF16 ? 1u : p.type == kQ4_0 ? 2u : 4u;   // kUnit
     s.steps_per_split = static_cast<std::uint32_t>(ceil_div(ceil_div(s.steps, splits), unit) * unit);
     s.splits = static_cast<std::uint32_t>(ceil_div(s.steps, s.steps_per_split));
     return s;
@@ -519,6 +678,7 @@ hipError_t launch_stream_linear(const TilePlanes& p, const SplitWorkspace& ws, c
     a.nt = p.nt;
     a.kt = p.kt;
     a.n = p.n;
+    a.k = p.k;
     a.xs = static_cast<const u32x4*>(ws.xs);
     a.blocks = static_cast<std::uint32_t>(p.kp / 32u);
     a.inv_scale = ws.inv_scale;
@@ -544,6 +704,11 @@ hipError_t launch_stream_linear(const TilePlanes& p, const SplitWorkspace& ws, c
     case kQ8_0: err = launch_fmt<kQ8_0>(a, shape, blocks, stream); break;
     case kQ4_0: err = launch_fmt<kQ4_0>(a, shape, blocks, stream); break;
     case kQ4_K: err = launch_fmt<kQ4_K>(a, shape, blocks, stream); break;
+    case kF16: err = launch_fmt<kF16>(a, shape, blocks, stream); break;
+    case kQ6_K:
+        a.scales = static_cast<const unsigned char*>(p.codes) + p.n * (p.k / 256u) * kQ6kRecord;
+        err = launch_fmt<kQ6_K>(a, shape, blocks, stream);
+        break;
     default: break;
     }
     if (err != hipSuccess || !split || chained) return err;

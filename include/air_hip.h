@@ -201,7 +201,10 @@ int air_hip_context_set_split_chain(air_hip_context* ctx, uint32_t mode);
  * the reference's batch-reuse matmul (src/cuda/cuda_backend.cu:529-583). */
 int air_hip_context_set_skinny_waves(air_hip_context* ctx, uint32_t waves);
 /* Chooses the decode kernel for 2..64 rows (autotuning): path 0 = automatic
- * (the skinny kernel: activations split once into the workspace and staged
+ * (while no other override of these widths is set, the streaming kernel
+ * wherever it measured faster: weights through registers, activations split
+ * once and brought into LDS by waves of their own; else the skinny kernel:
+ * activations split once into the workspace and staged
  * through LDS, every weight read once, K split over workgroups when the
  * weight tiles cannot fill the GPU), 1 = the single-launch fused kernel for
  * M <= 16 and the per-wave K-split kernel above, 2 = skinny.  tile_n = 16-row
@@ -229,7 +232,8 @@ int air_hip_context_set_decode_pipeline(air_hip_context* ctx, uint32_t lds_stage
 int air_hip_context_set_wsplit(air_hip_context* ctx, uint32_t mode, uint32_t tile_n, uint32_t waves, uint32_t depth,
                                uint32_t k_splits, uint32_t split_x);
 /* Chooses the kernel of the dense matrices (F16, BF16 and Q6_K storage;
- * autotuning): path 0 = automatic (the matrix-core kernel for 2..64 rows,
+ * autotuning): path 0 = automatic (for 2..64 rows the streaming kernel on
+ * F16 and Q6_K rows where it measured faster, else the matrix-core kernel;
  * the f16 prefill GEMM on the rows at prefill widths, FMA kernels
  * otherwise), 1 = the matrix-core kernel at every width, 2 = the FMA
  * kernels.

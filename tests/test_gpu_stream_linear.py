@@ -4,7 +4,7 @@ Shapes at the edges of its tiles: K an odd number of 64-k steps, a tail
 shorter than its chunks, K splits with a short last one, N not a multiple of
 16 and of a workgroup's row tiles, every count of activation tiles; wide
 matrices of one and two tiles per wave.  Each result is held to the oracle at
-relative L2 1e-4 per row, repeats to the same bits, and the no-allocation
+relative L2 1e-4 per row (1e-5 over dense rows), repeats to the same bits, and the no-allocation
 entry point to the same bits too.
 """
 import numpy as np
@@ -13,10 +13,12 @@ import pytest
 import oracle
 from air_amd import capi
 from tests import helpers
+from tests.test_gpu_dense import _weights
 
 pytestmark = pytest.mark.gpu
 
 DECODE_TOL = 1e-4
+DENSE_TOL = 1e-5          # the gate of the dense kernels
 
 # (format, K, N, widths)
 CASES = [
@@ -31,6 +33,12 @@ CASES = [
     (capi.TYPE_Q4_K, 2304, 4200, (20, 48)),
     (capi.TYPE_Q4_K, 8448, 1530, (2, 16, 17, 64)),
     (capi.TYPE_Q4_K, 2048, 41000, (7, 30, 64)),
+    (capi.TYPE_Q6_K, 2304, 4200, (3, 17, 33, 64)),    # dense rows: two splits of nine super-blocks
+    (capi.TYPE_Q6_K, 8448, 1530, (2, 16, 40)),
+    (capi.TYPE_Q6_K, 2048, 41000, (5, 20, 50)),
+    (capi.TYPE_F16, 3104, 4200, (17, 33, 64)),        # a row ends on the first block of a step
+    (capi.TYPE_F16, 8224, 1530, (18, 48)),
+    (capi.TYPE_F16, 2048, 41000, (24, 49)),
 ]
 
 
@@ -38,8 +46,10 @@ CASES = [
 def test_stream_linear(torch_cuda, hip_ctx, type_id, k, n, ms):
     torch = torch_cuda
     dev = torch.device("cuda:0")
-    canon = helpers.weights(type_id, k, n, seed=k + n)
+    dense = type_id in (capi.TYPE_Q6_K, capi.TYPE_F16)
+    canon = (_weights if dense else helpers.weights)(type_id, k, n, seed=k + n)
     mat = capi.Matrix(hip_ctx, type_id, k, n, canon, canon.nbytes, on_device=False)
+    tol = DENSE_TOL if dense else DECODE_TOL
     rows = np.unique(np.concatenate([np.arange(0, n, max(1, n // 200)), np.arange(max(0, n - 40), n)])).astype(np.uint64)
     bias = (np.random.default_rng(n).standard_normal(n) * 0.02).astype(np.float32)
     bias_d = torch.from_numpy(bias).to(dev)
@@ -68,7 +78,7 @@ def test_stream_linear(torch_cuda, hip_ctx, type_id, k, n, ms):
             want = oracle.linear_row_list(type_id, canon, k, n, x, rows, bias=bias)
             got = outs[0][:, rows.astype(np.int64)]
             for r in range(m):
-                assert helpers.rel_l2(got[r], want[r]) <= DECODE_TOL, (m, r, plan)
+                assert helpers.rel_l2(got[r], want[r]) <= tol, (m, r, plan)
     finally:
         mat.release()
 
