@@ -274,6 +274,13 @@ SkinnyShape plan_stream(const TilePlanes& planes, std::uint32_t m);
 hipError_t launch_stream_linear(const TilePlanes& planes, const SplitWorkspace& ws, const float* bias, float* y,
                                 std::uint32_t m, const SkinnyShape& shape, float* partials, hipStream_t stream,
                                 const SplitEpilogue* epilogue = nullptr, std::uint64_t* chain = nullptr);
+// The linear of a fused gate|up matrix with the SwiGLU in the same launch
+// (out [m][n / 2]), bit-identical to the linear of plan `linear` followed by
+// launch_silu_mul.  plan_stream_swiglu: whether it takes this one, and its
+// shape.
+bool plan_stream_swiglu(const TilePlanes& planes, std::uint32_t m, const SkinnyShape& linear, SkinnyShape& shape);
+hipError_t launch_stream_swiglu(const TilePlanes& planes, const SplitWorkspace& ws, const float* bias, float* out,
+                                std::uint32_t m, const SkinnyShape& shape, hipStream_t stream);
 // The same linear straight from f32 activations x [m][k]: each workgroup
 // splits the activations it stages (one power-of-two scale per (row,
 // 32-block)), so no split launch and no activation workspace.

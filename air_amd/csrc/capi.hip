@@ -443,7 +443,9 @@ Route route_linear(const air_hip_context* ctx, const air_hip_matrix* m, std::uin
 // loaded stay as they are.
 int run_stream(air_hip_context* ctx, const air_hip_matrix* m, const TilePlanes& planes, const float* x, float* y,
                const float* bias, std::uint32_t rows, const SplitEpilogue* epilogue, bool* applied, const void* ready) {
-    const SkinnyShape shape = plan_stream(planes, rows);
+    const SkinnyShape shape = skinny_plan(ctx, planes, rows);
+    SkinnyShape swiglu{};
+    const bool fused = epilogue && epilogue->kind == kEpilogueSwiglu && plan_stream_swiglu(planes, rows, shape, swiglu);
     const std::uint64_t kp = ceil_div(planes.k, kSplitK) * kSplitK;
     SplitWorkspace ws{};
     if (ready == x && ctx->loaded_k == planes.k && ctx->loaded_rows == rows && ctx->loaded_row_scaled) {
@@ -455,6 +457,14 @@ int run_stream(air_hip_context* ctx, const air_hip_matrix* m, const TilePlanes& 
         ws = carve_split_workspace(ctx->stream_rows, kp, rows);
         const hipError_t err = launch_split_activations_rows(x, rows, planes.k, kp, ws, ctx->stream);
         if (err != hipSuccess) return hip_fail(err, "split_rows_kernel");
+    }
+    if (fused) {
+        const hipError_t err = launch_stream_swiglu(planes, ws, bias, epilogue->out, rows, swiglu, ctx->stream);
+        if (err != hipSuccess) return hip_fail(err, "stream_kernel");
+        *applied = true;
+        ctx->decode_linear_calls.fetch_add(1, std::memory_order_relaxed);
+        ctx->decode_rows.fetch_add(rows, std::memory_order_relaxed);
+        return AIR_HIP_OK;
     }
     const std::uint64_t partial_bytes = skinny_partials_bytes(shape, rows, planes.n);
     if (partial_bytes > 0u) {
@@ -476,7 +486,12 @@ int run_stream(air_hip_context* ctx, const air_hip_matrix* m, const TilePlanes& 
 int run_skinny_x(air_hip_context* ctx, const air_hip_matrix* m, const float* x, float* y, const float* bias,
                  std::uint32_t rows, const SplitEpilogue* epilogue, bool* applied, const void* ready) {
     const SkinnyShape shape = skinny_plan(ctx, m->planes, rows);
-    if (shape.stream) return run_stream(ctx, m, m->planes, x, y, bias, rows, epilogue, applied, ready);
+    // The streaming kernel, or a SwiGLU it takes off the eight-wave kernel's hands.
+    SkinnyShape swiglu{};
+    if (shape.stream || (decode_automatic(ctx) && epilogue && epilogue->kind == kEpilogueSwiglu &&
+                         plan_stream_swiglu(m->planes, rows, shape, swiglu))) {
+        return run_stream(ctx, m, m->planes, x, y, bias, rows, epilogue, applied, ready);
+    }
     if (skinny_route(ctx, m, rows) == Route::skinny_loaded) {
         int rc = load_activations_for(ctx, x, m->planes.k, rows, ready);
         if (rc != AIR_HIP_OK) return rc;

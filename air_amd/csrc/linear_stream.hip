@@ -1,6 +1,7 @@
 // linear_stream.hip -- the decode linear for M = 2..64 rows over split
-// activations, in the tile formats and over dense F16 and Q6_K rows: weights streamed through registers, activations shared through
-// LDS by waves that do nothing else.
+// activations, in the tile formats and over dense F16 and Q6_K rows: weights
+// streamed through registers, activations shared through LDS by waves that do
+// nothing else.
 //
 // The arithmetic of skinny_kernel / skinny_lds_kernel (linear_skinny.hip);
 // what differs is how the operands travel:
@@ -91,7 +92,18 @@ struct StreamArgs {
     float* y;
     const float* chain_bias;
     std::uint32_t splits;
+    // SWIGLU: the matrix is a fused gate|up of 2 * ffn_tiles row tiles and out
+    // is [m][n / 2].  serial: K splits one workgroup sums itself, in order.
+    std::uint32_t ffn_tiles;
+    std::uint32_t serial;
 };
+
+// silu(g) * u in silu_mul_kernel's arithmetic (no fused products).
+__device__ __forceinline__ float swiglu(float g, float u) {
+#pragma clang fp contract(off)
+    const float s = g / (1.0f + expf(-g));
+    return s * u;
+}
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) void global_void_t;
@@ -253,13 +265,23 @@ constexpr unsigned kLevels = FMT == kF16 && MT == 2 && TN == 2 ? 2u
                              : FMT == kQ4_K || (MT == 4 && TN == 2) ? 1u
                                                                     : 2u;
 
-template <int FMT, int MT, int TN, int W>
+// SWIGLU: the workgroup's tiles are W * TN / 2 gate tiles and the up tiles
+// that belong to them (TN = 2: both in one wave; else waves w and w + W / 2,
+// which meet in LDS), and it stores silu(gate) * up: the SwiGLU launch and
+// its round trip through the fused rows go away.  7B gate|up with its SwiGLU,
+// graph replay: at 32 rows Q8_0 46.2 -> 37.4 us (eight-wave kernel and its
+// reduction before), Q4_0 44.8 -> 32.3, Q4_K 51.0 -> 38.8; at 64 65.7 -> 54.7,
+// 67.6 -> 51.1, 81.4 -> 59.5 (the streaming kernel's share included).
+// SERIAL: the K splits of a plan that sums them in a reduction, one after the
+// other in one workgroup: each in one running sum, scaled, then added from
+// zero in split order -- that plan's bits.
+template <int FMT, int MT, int TN, int W, bool SWIGLU, bool SERIAL>
 __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) void stream_kernel(StreamArgs a) {
     constexpr unsigned P = kProducers;
     constexpr unsigned U = kUnit<FMT>;
     constexpr unsigned D = kRing<FMT, MT, TN>;
     constexpr unsigned C = kChunk<MT>;
-    constexpr unsigned L = kLevels<FMT, MT, TN>;
+    constexpr unsigned L = SERIAL ? 1u : kLevels<FMT, MT, TN>;
     // Steps per trip: the ring comes full circle.  At three levels the second
     // one covers eight steps (two trips of four with four activation tiles,
     // which would spill in a trip of eight).
@@ -283,9 +305,15 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
     const std::uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const std::uint32_t group = blockIdx.x % a.groups;
     const std::uint32_t split = blockIdx.x / a.groups;
-    const std::uint32_t rt0 = (group * W + wave) * TN;
-    const std::uint32_t s_begin = split * a.steps_per_split;
-    const std::uint32_t s_end = min(a.steps, s_begin + a.steps_per_split);
+    const std::uint32_t range = a.steps_per_split * (SERIAL ? a.serial : 1u);
+    const std::uint32_t s_begin = split * range;
+    const std::uint32_t s_end = min(a.steps, s_begin + range);
+    // Row tile j of the wave.
+    const auto row_tile = [&](int j) __attribute__((always_inline)) -> std::uint32_t {
+        if constexpr (!SWIGLU) return (group * W + wave) * TN + static_cast<std::uint32_t>(j);
+        else if constexpr (TN == 2) return group * W + wave + (j != 0 ? a.ffn_tiles : 0u);
+        else return wave < W / 2 ? group * (W / 2) + wave : a.ffn_tiles + group * (W / 2) + wave - W / 2;
+    };
     const std::uint32_t chunk_count = (s_end - s_begin + C - 1u) / C;   // ranges are never empty
 
     if (wave >= W) {
@@ -335,9 +363,9 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
         if constexpr (kDense) {   // the lane's row
-            wtile[j] = min(static_cast<std::uint64_t>(rt0 + static_cast<std::uint32_t>(j)) * 16u + (lane & 15u), a.n - 1u);
+            wtile[j] = min(static_cast<std::uint64_t>(row_tile(j)) * 16u + (lane & 15u), a.n - 1u);
         } else {
-            wtile[j] = static_cast<std::uint64_t>(min(rt0 + static_cast<std::uint32_t>(j), a.nt - 1u)) * a.kt;
+            wtile[j] = static_cast<std::uint64_t>(min(row_tile(j), a.nt - 1u)) * a.kt;
         }
     }
     Record<FMT> ring[D][TN];
@@ -480,6 +508,31 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
         load_w(ring[d.value], s_begin / U + d.value);
         __builtin_amdgcn_sched_barrier(0);   // the loop's load counting needs this order too
     });
+    float4v inv[MT];
+    const auto load_inv = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) inv[t] = reinterpret_cast<const float4v*>(a.inv_scale)[t * 4 + (lane >> 4)];
+    };
+    float4v total[SERIAL ? TN : 1][SERIAL ? MT : 1];
+    std::uint32_t flush = s_begin + a.steps_per_split;
+    const auto flush_split = [&]() __attribute__((always_inline)) {
+#pragma clang fp contract(off)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                total[SERIAL ? j : 0][SERIAL ? t : 0] += acc[j][t] * inv[t];
+                acc[j][t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        flush += a.steps_per_split;
+    };
+    if constexpr (SERIAL) {
+        load_inv();
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) total[j][t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    }
     // One trip: kBody steps from s.  WHOLE: all of them lie in the range.
     std::uint32_t buffer = 0u;
     bool first_half = true;   // kHold: of the second level's eight steps
@@ -508,6 +561,9 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
                 read_stage.template operator()<0>(cur);
             }
             if (WHOLE || s + i < s_end) {
+                if constexpr (SERIAL) {
+                    if (s + i == flush) flush_split();
+                }
                 compute.template operator()<2u * cs, i % U, 0, false>(cur, ring[(i / U) % D]);
                 compute.template operator()<2u * cs + 1u, i % U, 1, cs + 1u == C>(cur, ring[(i / U) % D]);
             }
@@ -539,14 +595,53 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
     }
 
     // D[row = activation row][col = weight row], as skinny_kernel.
-    float4v inv[MT];
+    if constexpr (SERIAL) flush_split();
+    else load_inv();
+    const auto value = [&](int j, int t, int i, float bn) __attribute__((always_inline)) {
+        if constexpr (SERIAL) return total[j][t][i] + bn;
+        else return acc[j][t][i] * inv[t][i] + bn;
+    };
+    if constexpr (SWIGLU) {
+        __shared__ float4v up_rows[TN == 2 ? 1 : W / 2][MT][64];
+        const std::uint64_t ffn = a.n / 2u;
+        const std::uint64_t n = static_cast<std::uint64_t>(row_tile(0)) * 16u + (lane & 15u);   // gate (or up) row
+        const bool is_up = TN == 1 && wave >= W / 2;
+        const bool live = n < (is_up ? a.n : ffn);
+        const float b0 = a.bias && live ? a.bias[n] : 0.0f;
+        if constexpr (TN == 1) {
+            if (is_up) {
 #pragma unroll
-    for (int t = 0; t < MT; ++t) inv[t] = reinterpret_cast<const float4v*>(a.inv_scale)[t * 4 + (lane >> 4)];
+                for (int t = 0; t < MT; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) up_rows[wave - W / 2][t][lane][i] = value(0, t, i, b0);
+            }
+            lds_barrier();
+            if (is_up) return;
+        }
+        if (!live) return;
+        const float b1 = TN == 2 && a.bias ? a.bias[ffn + n] : 0.0f;
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            float4v u;
+            if constexpr (TN == 2) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) u[i] = value(TN - 1, t, i, b1);
+            } else {
+                u = up_rows[wave][t][lane];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const std::uint32_t m = static_cast<std::uint32_t>(t) * 16u + 4u * (lane >> 4) + static_cast<std::uint32_t>(i);
+                if (m < a.m) a.out[static_cast<std::uint64_t>(m) * ffn + n] = swiglu(value(0, t, i, b0), u[i]);
+            }
+        }
+        return;
+    }
     float* out = a.out + (a.partial ? static_cast<std::uint64_t>(split) * a.m * a.n : 0u);
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-        const std::uint64_t n = static_cast<std::uint64_t>(rt0 + static_cast<std::uint32_t>(j)) * 16u + (lane & 15u);
-        if (rt0 + static_cast<std::uint32_t>(j) >= a.nt || n >= a.n) continue;
+        const std::uint64_t n = static_cast<std::uint64_t>(row_tile(j)) * 16u + (lane & 15u);
+        if (row_tile(j) >= a.nt || n >= a.n) continue;
         const float bn = a.bias ? a.bias[n] : 0.0f;
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
@@ -555,7 +650,7 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
                 const std::uint32_t m = static_cast<std::uint32_t>(t) * 16u + 4u * (lane >> 4) + static_cast<std::uint32_t>(i);
                 if (m >= a.m) continue;
                 const std::uint64_t e = static_cast<std::uint64_t>(m) * a.n + n;
-                float v = acc[j][t][i] * inv[t][i] + bn;
+                float v = value(j, t, i, bn);
                 if (a.chain) {
                     if (chain_combine(a.chain, static_cast<std::uint64_t>(a.m) * a.n, e, split, a.splits, v)) {
                         a.y[e] = a.chain_bias ? v + a.chain_bias[n] : v;
@@ -570,7 +665,20 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
 
 template <int FMT, int MT, int TN, int W>
 hipError_t launch_w(const StreamArgs& a, std::uint32_t blocks, hipStream_t stream) {
-    hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W>), dim3(blocks), dim3(64 * (W + kProducers)), 0, stream, a);
+    const dim3 threads(64 * (W + kProducers));
+    if (a.ffn_tiles == 0u) {
+        hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, false, false>), dim3(blocks), threads, 0, stream, a);
+    } else if constexpr (dense_storage(FMT)) {
+        return hipErrorInvalidConfiguration;
+    } else if (a.serial > 1u) {
+        if constexpr (FMT == kQ8_0 && MT == 2 && W == 10) {
+            hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, true, true>), dim3(blocks), threads, 0, stream, a);
+        } else {
+            return hipErrorInvalidConfiguration;
+        }
+    } else {
+        hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, true, false>), dim3(blocks), threads, 0, stream, a);
+    }
     return hipGetLastError();
 }
 
@@ -666,13 +774,13 @@ SkinnyShape plan_stream(const TilePlanes& p, std::uint32_t m) {
     return s;
 }
 
-hipError_t launch_stream_linear(const TilePlanes& p, const SplitWorkspace& ws, const float* bias, float* y,
-                                std::uint32_t m, const SkinnyShape& shape, float* partials, hipStream_t stream,
-                                const SplitEpilogue* epilogue, std::uint64_t* chain) {
-    if (m == 0u || m > 64u || shape.mt != ceil_div(m, 16u) || shape.steps == 0u || shape.steps_per_split == 0u) {
+namespace {
+
+hipError_t launch_stream(const TilePlanes& p, const SplitWorkspace& ws, StreamArgs a, std::uint32_t m,
+                         const SkinnyShape& s, hipStream_t stream) {
+    if (m == 0u || m > 64u || s.mt != ceil_div(m, 16u) || s.steps == 0u || s.steps_per_split == 0u) {
         return hipErrorInvalidValue;
     }
-    StreamArgs a{};
     a.codes = p.codes;
     a.scales = p.scales;
     a.nt = p.nt;
@@ -684,9 +792,29 @@ hipError_t launch_stream_linear(const TilePlanes& p, const SplitWorkspace& ws, c
     a.inv_scale = ws.inv_scale;
     a.block_sums = ws.block_sums;
     a.m = m;
-    a.groups = shape.groups;
-    a.steps = shape.steps;
-    a.steps_per_split = shape.steps_per_split;
+    a.groups = s.groups;
+    a.steps = s.steps;
+    a.steps_per_split = s.steps_per_split;
+    const std::uint32_t blocks = s.groups * (a.serial > 1u ? 1u : s.splits);
+    switch (p.type) {
+    case kQ8_0: return launch_fmt<kQ8_0>(a, s, blocks, stream);
+    case kQ4_0: return launch_fmt<kQ4_0>(a, s, blocks, stream);
+    case kQ4_K: return launch_fmt<kQ4_K>(a, s, blocks, stream);
+    case kF16: return launch_fmt<kF16>(a, s, blocks, stream);
+    case kQ6_K:
+        a.scales = static_cast<const unsigned char*>(p.codes) + p.n * (p.k / 256u) * kQ6kRecord;
+        return launch_fmt<kQ6_K>(a, s, blocks, stream);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+} // namespace
+
+hipError_t launch_stream_linear(const TilePlanes& p, const SplitWorkspace& ws, const float* bias, float* y,
+                                std::uint32_t m, const SkinnyShape& shape, float* partials, hipStream_t stream,
+                                const SplitEpilogue* epilogue, std::uint64_t* chain) {
+    StreamArgs a{};
+    a.serial = 1u;
     const bool split = shape.splits > 1u;
     const bool chained = split && chain && !epilogue;
     a.partial = split ? 1u : 0u;
@@ -698,22 +826,42 @@ hipError_t launch_stream_linear(const TilePlanes& p, const SplitWorkspace& ws, c
         a.chain_bias = bias;
         a.splits = shape.splits;
     }
-    const std::uint32_t blocks = shape.groups * shape.splits;
-    hipError_t err = hipErrorInvalidValue;
-    switch (p.type) {
-    case kQ8_0: err = launch_fmt<kQ8_0>(a, shape, blocks, stream); break;
-    case kQ4_0: err = launch_fmt<kQ4_0>(a, shape, blocks, stream); break;
-    case kQ4_K: err = launch_fmt<kQ4_K>(a, shape, blocks, stream); break;
-    case kF16: err = launch_fmt<kF16>(a, shape, blocks, stream); break;
-    case kQ6_K:
-        a.scales = static_cast<const unsigned char*>(p.codes) + p.n * (p.k / 256u) * kQ6kRecord;
-        err = launch_fmt<kQ6_K>(a, shape, blocks, stream);
-        break;
-    default: break;
-    }
+    const hipError_t err = launch_stream(p, ws, a, m, shape, stream);
     if (err != hipSuccess || !split || chained) return err;
     if (epilogue) return launch_split_epilogue(partials, shape.splits, m, p.n, bias, *epilogue, stream);
     return launch_split_reduce(partials, shape.splits, m, p.n, bias, y, stream);
+}
+
+bool plan_stream_swiglu(const TilePlanes& p, std::uint32_t m, const SkinnyShape& linear, SkinnyShape& s) {
+    if (dense_storage(p.type) || p.n % 32u != 0u || m < 2u || m > 64u) return false;
+    const std::uint32_t ffn_tiles = p.nt / 2u;
+    if (linear.stream) {
+        // The linear's own workgroups, with half gate and half up tiles; a K
+        // split goes through the reduction, which carries the SwiGLU.
+        if (linear.splits != 1u) return false;
+        s = linear;
+    } else {
+        // Q8_0 at 17..32 rows, 2000..4096 row tiles: the plain linear keeps
+        // the eight-wave kernel (37.8 us; its two splits reduce in another
+        // 5 with the SwiGLU); here its splits are summed in the workgroup.
+        if (p.type != kQ8_0 || m <= 16u || m > 32u || p.nt < 2000u || p.nt > 4096u || p.kp / kStepK < 32u) return false;
+        s = linear;
+        s.stream = true;
+        s.waves = 10u;
+        s.tile_n = p.nt > 2560u ? 2u : 1u;
+    }
+    s.groups = static_cast<std::uint32_t>(ceil_div(ffn_tiles, s.waves * s.tile_n / 2u));
+    return true;
+}
+
+hipError_t launch_stream_swiglu(const TilePlanes& p, const SplitWorkspace& ws, const float* bias, float* out,
+                                std::uint32_t m, const SkinnyShape& s, hipStream_t stream) {
+    StreamArgs a{};
+    a.serial = s.splits;
+    a.ffn_tiles = p.nt / 2u;
+    a.bias = bias;
+    a.out = out;
+    return launch_stream(p, ws, a, m, s, stream);
 }
 
 } // namespace air_hip

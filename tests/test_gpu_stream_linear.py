@@ -108,3 +108,54 @@ def test_stream_outliers_keep_small_channels(torch_cuda, hip_ctx):
             assert np.linalg.norm(got[r] - want[r]) <= 1e-3 * np.linalg.norm(share[r]), r
     finally:
         mat.release()
+
+
+# (format, K, N of the fused gate|up, widths): one and two tiles per wave,
+# eight waves, a last workgroup short of tiles, an odd count of gate tiles;
+# the Q8_0 rows at 2000..4096 row tiles and 17..32 rows sum their two K splits
+# in one workgroup (33 steps: unequal halves).
+SWIGLU_CASES = [
+    (capi.TYPE_Q8_0, 2112, 32 * 1001, (17, 32)),
+    (capi.TYPE_Q8_0, 2048, 32 * 1301, (2, 16, 20, 31, 64)),
+    (capi.TYPE_Q8_0, 2112, 32 * 997, (5, 40)),
+    (capi.TYPE_Q8_0, 3616, 32 * 2048, (25, 49)),
+    (capi.TYPE_Q4_0, 2048, 32 * 1301, (3, 18, 33, 64)),
+    (capi.TYPE_Q4_0, 2112, 32 * 999, (16, 47)),
+    (capi.TYPE_Q4_K, 2304, 32 * 1283, (9, 32, 64)),
+    (capi.TYPE_Q4_K, 2304, 32 * 1033, (16, 48)),
+]
+
+
+@pytest.mark.parametrize("type_id,k,n,ms", SWIGLU_CASES,
+                         ids=[f"{capi.TYPE_NAMES[c[0]]}-{c[2]}x{c[1]}" for c in SWIGLU_CASES])
+def test_stream_swiglu_bits(torch_cuda, hip_ctx, type_id, k, n, ms):
+    """The SwiGLU in the linear's launch: the bits of the linear followed by
+    air_hip_silu_mul, and no write past the output."""
+    torch = torch_cuda
+    lib = capi.lib()
+    h = hip_ctx.handle
+    f = n // 2
+    canon = helpers.weights(type_id, k, n, seed=k + n)
+    mat = capi.Matrix(hip_ctx, type_id, k, n, canon, canon.nbytes, on_device=False)
+    bias = torch.from_numpy((np.random.default_rng(n).standard_normal(n) * 0.3).astype(np.float32)).to("cuda:0")
+    try:
+        for m in ms:
+            x = helpers.activations(m, k, seed=m + k)
+            x[:, ::61] *= 40.0
+            x[m // 2] *= 1e-5
+            xd = torch.from_numpy(x).to("cuda:0")
+            for b in (None, bias):
+                bp = b.data_ptr() if b is not None else None
+                lin = torch.empty((m, n), dtype=torch.float32, device="cuda:0")
+                want = torch.empty((m, f), dtype=torch.float32, device="cuda:0")
+                capi.check(lib.air_hip_linear(h, mat.handle, xd.data_ptr(), lin.data_ptr(), bp, m, capi.LINEAR_DECODE))
+                capi.check(lib.air_hip_silu_mul(h, lin.data_ptr(), want.data_ptr(), m, f))
+                got = torch.full((m + 1, f), -7.0, dtype=torch.float32, device="cuda:0")
+                capi.check(lib.air_hip_linear_epilogue(h, mat.handle, xd.data_ptr(), m, got.data_ptr(), bp,
+                                                       capi.EPILOGUE_SWIGLU, None, None, 0.0, capi.LINEAR_DECODE))
+                torch.cuda.synchronize()
+                case = (m, b is not None, mat.plan(m))
+                assert np.array_equal(got[:m].cpu().numpy().view(np.uint32), want.cpu().numpy().view(np.uint32)), case
+                assert bool((got[m] == -7.0).all()), case
+    finally:
+        mat.release()
