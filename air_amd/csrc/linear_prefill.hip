@@ -883,8 +883,8 @@ PrefillShape plan_prefill(const TilePlanes& p, std::uint32_t m, const PrefillTun
     PrefillShape s;
     // Register tile per wave: TM x TN MFMA tiles (16 x 16 each).  Measured on
     // the Qwen2-7B shapes at M = 512 (TFLOP/s, Q8_0 / Q4_0 / Q4_K):
-    //  * long K (down, K = 18944): 8x4, one step of prefetch, 8 K splits
-    //    (623 / 649 / 571; 8x2 with 4 splits 612 / 632 / 562);
+    //  * long K (down, K = 18944): 8x4, one step of prefetch (at
+    //    8 K splits 623 / 649 / 571; 8x2 with 4 splits 612 / 632 / 562);
     //  * wide grids (gate|up, 2368 row tiles): Q8_0 8x4 with one step of
     //    prefetch (694; 8x2 663), the 4-bit formats 8x2 (805 / 708; 8x4
     //    703 / 550) -- their codes are half the bytes, so the shorter
@@ -922,12 +922,36 @@ PrefillShape plan_prefill(const TilePlanes& p, std::uint32_t m, const PrefillTun
     std::uint32_t splits = tuning.k_splits;
     if (splits == 0u) {
         // Split K while the doubled grid stays within 2.5 workgroups per CU,
-        // keeping at least 16 steps per split: q|k|v (288 tiles) and o (224)
-        // split 2 ways, down (56) 8 ways (measured: q|k|v 4 ways 4 % and o
-        // 4 ways 1 % off their best; down 16 ways 16 % slower).
+        // keeping at least 16 steps per split (Q8_0 q|k|v at M = 512: 288
+        // tiles, 43.5 us split 2 ways, 50.5 unsplit).
         const std::uint64_t tiles = static_cast<std::uint64_t>(s.m_tiles) * s.groups;
+        const std::uint64_t cus = tuning.cus ? tuning.cus : 256u, slots = 2u * cus;
         splits = 1u;
         while (tiles * splits * 2u <= 640u && s.steps / (splits * 2u) >= 16u) splits *= 2u;
+        if (s.tile_m == 4u && s.tile_n == 2u) {
+            // Fewer row tiles leave room for more: up to two workgroups per
+            // CU, at least 14 steps each.  o (28 groups) at M = 96, 160, 256
+            // and 301: Q8_0 27.5 -> 21.7, 29.2 -> 25.6, 31.2 -> 27.7 and
+            // 33.3 -> 29.8 us, Q4_K 39.9 -> 34.8 at 301; six splits are no
+            // better than four at 96 (22.3).
+            splits = std::max<std::uint32_t>(splits, static_cast<std::uint32_t>(std::min<std::uint64_t>(slots / tiles, s.steps / 14u)));
+        } else if (s.tile_m == 8u && s.tile_n == 4u && tiles <= slots) {
+            // At most the two workgroups a CU holds, and of those counts the
+            // one whose last workgroup per CU is missing least often: down
+            // (14 groups) at M = 96 takes 18 splits (252 workgroups; Q8_0
+            // 51.3 -> 48.0 us, 20 splits 53.2), at 301 12 (504; 91.6 -> 81.8,
+            // Q4_K 102.1 -> 88.1), at 512 9 (101.1 -> 99.8, 10 splits 141).
+            // More tiles than CUs stay whole: gate|up at 256 rows paid for
+            // 78 MB of partials.
+            std::uint64_t best = 0u;
+            for (std::uint64_t n = 1u; tiles * n <= slots && (n == 1u || s.steps / n >= 16u); ++n) {
+                const std::uint64_t fill = tiles * n * 1024u / (ceil_div(tiles * n, cus) * cus);
+                if (fill >= best) {
+                    best = fill;
+                    splits = static_cast<std::uint32_t>(n);
+                }
+            }
+        }
     }
     // A grid of 8x4 tiles (two workgroups per CU) that ends in a round less
     // than half full -- Qwen2-7B gate|up at M = 512: 592 workgroups on 512

@@ -507,3 +507,37 @@ def test_prefill_residual_epilogues(torch_cuda, hip_ctx, k, n, m, splits):
         hip_ctx.set_prefill_tuning(0, 0, 0, 0)
         mat.release()
         mat2.release()
+
+
+# K splits that fill the CUs' workgroup slots: (format, K, N, M, splits): odd
+# counts on the 4x2 tile, a short last split, the 8x4 tile's 12 and 18, and
+# more tiles than CUs unsplit.
+SPLIT_CASES = [
+    (capi.TYPE_Q8_0, 3584, 3571, 96, 4),
+    (capi.TYPE_Q4_K, 2816, 3584, 301, 3),
+    (capi.TYPE_Q4_0, 4160, 2100, 70, 4),
+    (capi.TYPE_Q8_0, 18944, 3584, 301, 12),
+    (capi.TYPE_Q4_K, 18944, 3571, 96, 18),
+    (capi.TYPE_Q8_0, 1024, 37888, 160, 1),
+]
+
+
+@pytest.mark.parametrize("type_id,k,n,m,splits", SPLIT_CASES)
+def test_prefill_fill_splits(torch_cuda, hip_ctx, type_id, k, n, m, splits):
+    torch = torch_cuda
+    canon = helpers.weights(type_id, k, n, seed=k + n)
+    mat = capi.Matrix(hip_ctx, type_id, k, n, canon, canon.nbytes, on_device=False)
+    bias = np.random.default_rng(n).standard_normal(n).astype(np.float32) * 0.02
+    x = helpers.activations(m, k, seed=m + k)
+    rows = np.unique(np.concatenate([np.arange(0, n, n // 50), np.arange(n - 20, n)])).astype(np.uint64)
+    sample = np.array([0, m // 2, m - 1])
+    try:
+        plan = mat.plan(m, tactic=capi.LINEAR_PREFILL)
+        print(f"fill {capi.TYPE_NAMES[type_id]} {n}x{k} M={m}: {plan}", flush=True)
+        assert plan.split(" + ")[0].endswith(f"splits={splits}"), plan
+        got = _run(torch, mat, x, n, m, bias)
+        assert np.array_equal(got, _run(torch, mat, x, n, m, bias))
+        want = oracle.linear_row_list(type_id, canon, k, n, x[sample], rows, bias=bias)
+        assert helpers.rel_l2(got[sample][:, rows.astype(np.int64)], want) < PREFILL_EXPECT, plan
+    finally:
+        mat.release()
