@@ -940,17 +940,19 @@ PrefillShape plan_prefill(const TilePlanes& p, std::uint32_t m, const PrefillTun
             // one whose last workgroup per CU is missing least often: down
             // (14 groups) at M = 96 takes 18 splits (252 workgroups; Q8_0
             // 51.3 -> 48.0 us, 20 splits 53.2), at 301 12 (504; 91.6 -> 81.8,
-            // Q4_K 102.1 -> 88.1), at 512 9 (101.1 -> 99.8, 10 splits 141).
-            // More tiles than CUs stay whole: gate|up at 256 rows paid for
-            // 78 MB of partials.
-            std::uint64_t best = 0u;
-            for (std::uint64_t n = 1u; tiles * n <= slots && (n == 1u || s.steps / n >= 16u); ++n) {
-                const std::uint64_t fill = tiles * n * 1024u / (ceil_div(tiles * n, cus) * cus);
-                if (fill >= best) {
-                    best = fill;
-                    splits = static_cast<std::uint32_t>(n);
-                }
+            // Q4_K 102.1 -> 88.1).  A power of two that already gives every CU
+            // a workgroup stays unless the other count fills a quarter more of
+            // the slots: at 512 rows 9 splits (504 workgroups) took 99.8 us, 8
+            // (448) 101.1, for an eighth more partials.  More tiles than CUs
+            // stay whole: gate|up at 256 rows paid for 78 MB of partials.
+            const auto fill = [&](std::uint64_t n) { return tiles * n * 1024u / (ceil_div(tiles * n, cus) * cus); };
+            const std::uint64_t power = splits;
+            std::uint64_t best = 1u;
+            for (std::uint64_t n = 2u; tiles * n <= slots && s.steps / n >= 16u; ++n) {
+                if (fill(n) >= fill(best)) best = n;
             }
+            const bool covers = tiles * power <= slots && tiles * power >= cus;
+            splits = static_cast<std::uint32_t>(covers && fill(best) * 4u <= fill(power) * 5u ? power : best);
         }
     }
     // A grid of 8x4 tiles (two workgroups per CU) that ends in a round less

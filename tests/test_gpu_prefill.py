@@ -517,6 +517,7 @@ SPLIT_CASES = [
     (capi.TYPE_Q4_K, 2816, 3584, 301, 3),
     (capi.TYPE_Q4_0, 4160, 2100, 70, 4),
     (capi.TYPE_Q8_0, 18944, 3584, 301, 12),
+    (capi.TYPE_Q8_0, 18944, 3584, 512, 8),     # every CU busy at a power of two: it stays
     (capi.TYPE_Q4_K, 18944, 3571, 96, 18),
     (capi.TYPE_Q8_0, 1024, 37888, 160, 1),
 ]
