@@ -1714,7 +1714,10 @@ int air_hip_linear_epilogue(air_hip_context* ctx, const air_hip_matrix* m, const
     if (rc != AIR_HIP_OK) return rc;
     if (prefill_out) {
         if (applied) {
-            remember_prefill(ctx, norm_out, n, rows);
+            // A reduction that could not carry the operand (a dense matrix, a
+            // decode route, an operand that would reach the partials) left
+            // another linear's in the workspace: the next linear converts.
+            if (e.prefill) remember_prefill(ctx, norm_out, n, rows);
             return AIR_HIP_OK;
         }
         // The linear wrote y: the residual add and the norm with the operand.

@@ -424,7 +424,10 @@ int air_hip_decode_linear_fused(air_hip_context* ctx, const air_hip_matrix* matr
  *   AIR_HIP_EPILOGUE_RESIDUAL_PREFILL: RESIDUAL with its norm (required), and
  *     norm_out is also converted for the next prefill linear as
  *     air_hip_rms_norm_prefill converts it, with the same reuse rules.
- *     Prefill-width linears with a K split carry it in their reduction.
+ *     Prefill-width linears of the tile formats with a K split carry it in
+ *     their reduction where the operand ends before the partials (n no wider
+ *     than k, in whole rows of the operand); a K split that carries the norm
+ *     without it leaves the conversion to the next linear.
  * Bit-identical to air_hip_linear (same tactic) followed by that call.  Where
  * the linear runs with a K split (a skinny launch at decode widths 2..64,
  * or a prefill GEMM), its split reduction

@@ -11,12 +11,15 @@ compiled launch shape and K splits.
 """
 from __future__ import annotations
 
+import re
+
 import numpy as np
 import pytest
 
 import oracle
 from air_amd import capi, quant
 from tests import helpers
+from tests.test_gpu_dense import _weights as dense_weights
 
 pytestmark = pytest.mark.gpu
 
@@ -505,6 +508,68 @@ def test_prefill_residual_epilogues(torch_cuda, hip_ctx, k, n, m, splits):
                                            capi.EPILOGUE_RESIDUAL_PREFILL, None, None, 0.0, pf) == 1
     finally:
         hip_ctx.set_prefill_tuning(0, 0, 0, 0)
+        mat.release()
+        mat2.release()
+
+
+# (format, K, N, M, tactic): a K split whose reduction carries the norm but not
+# the next linear's f16 operand -- dense rows at prefill and decode widths, tile
+# formats on a decode route, and an output too wide for its operand to end
+# before the partials.
+OPERAND_CASES = [
+    (capi.TYPE_F16, 1792, 1792, 65, capi.LINEAR_PREFILL),
+    (capi.TYPE_F16, 3584, 3584, 129, capi.LINEAR_AUTO),
+    (capi.TYPE_Q6_K, 1792, 1792, 65, capi.LINEAR_PREFILL),
+    (capi.TYPE_Q6_K, 3584, 3584, 301, capi.LINEAR_PREFILL),
+    (capi.TYPE_Q6_K, 8448, 1536, 8, capi.LINEAR_DECODE),
+    (capi.TYPE_F16, 8448, 1536, 24, capi.LINEAR_DECODE),
+    (capi.TYPE_Q8_0, 8448, 1536, 24, capi.LINEAR_DECODE),
+    (capi.TYPE_Q4_K, 8448, 1536, 8, capi.LINEAR_DECODE),
+    (capi.TYPE_Q8_0, 2048, 3584, 70, capi.LINEAR_PREFILL),
+]
+
+
+@pytest.mark.parametrize("type_id,k,n,m,tactic", OPERAND_CASES)
+def test_residual_prefill_without_operand(torch_cuda, hip_ctx, type_id, k, n, m, tactic):
+    """RESIDUAL_PREFILL followed by a prefill linear on norm_out: the bits of
+    the linear, air_hip_add_rms_norm and the prefill linear one by one."""
+    torch = torch_cuda
+    lib = capi.lib()
+    h = hip_ctx.handle
+    dense = type_id in (capi.TYPE_F16, capi.TYPE_Q6_K)
+    canon = (dense_weights if dense else helpers.weights)(type_id, k, n, seed=k + n + 29)
+    mat = capi.Matrix(hip_ctx, type_id, k, n, canon, canon.nbytes, on_device=False)
+    canon2 = helpers.weights(capi.TYPE_Q8_0, n, 640, seed=n + 31)
+    mat2 = capi.Matrix(hip_ctx, capi.TYPE_Q8_0, n, 640, canon2, canon2.nbytes, on_device=False)
+
+    def bits(t):
+        return t.cpu().numpy().view(np.uint32)
+
+    try:
+        plan = mat.plan(m, tactic=tactic)
+        print(f"operand {capi.TYPE_NAMES[type_id]} {n}x{k} M={m}: {plan}", flush=True)
+        assert int(re.search(r" splits=(\d+)", plan).group(1)) > 1, plan
+        x = _dev(torch, helpers.activations(m, k, seed=m + k))
+        resid = _dev(torch, helpers.activations(m, n, seed=m + 7))
+        resid_ref = resid.clone()
+        w = _dev(torch, helpers.activations(1, n, seed=k + 2)[0])
+        lin, normed_ref = (torch.empty((m, n), dtype=torch.float32, device="cuda:0") for _ in range(2))
+        normed = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda:0")
+        y2, y2_ref = (torch.empty((m, 640), dtype=torch.float32, device="cuda:0") for _ in range(2))
+        capi.check(lib.air_hip_linear(h, mat.handle, x.data_ptr(), lin.data_ptr(), None, m, tactic))
+        capi.check(lib.air_hip_add_rms_norm(h, resid_ref.data_ptr(), lin.data_ptr(), w.data_ptr(),
+                                            normed_ref.data_ptr(), m, n, 1e-6))
+        mat2.linear(normed_ref, y2_ref, m, tactic=capi.LINEAR_PREFILL)
+        mat2.linear(lin, y2, m, tactic=capi.LINEAR_PREFILL)      # another operand in the workspace
+        capi.check(lib.air_hip_linear_epilogue(h, mat.handle, x.data_ptr(), m, resid.data_ptr(), None,
+                                               capi.EPILOGUE_RESIDUAL_PREFILL, w.data_ptr(), normed.data_ptr(),
+                                               1e-6, tactic))
+        mat2.linear(normed, y2, m, tactic=capi.LINEAR_PREFILL)
+        torch.cuda.synchronize()
+        assert np.array_equal(bits(resid), bits(resid_ref)), plan
+        assert np.array_equal(bits(normed), bits(normed_ref)), plan
+        assert np.array_equal(bits(y2), bits(y2_ref)), plan
+    finally:
         mat.release()
         mat2.release()
 
