@@ -180,15 +180,18 @@ __device__ __forceinline__ void split8(const float (&v)[8], float s, half8v& hi,
 __device__ __forceinline__ void emit_split_run(std::uint64_t r, const float (&v)[8], float s, std::uint32_t m,
                                                std::uint32_t mp, uint4* __restrict__ xs,
                                                float* __restrict__ block_sums) {
+#pragma clang fp contract(off)
     const std::uint32_t mtiles = mp / 16u;
     const std::uint64_t b = r >> 2;
     const std::uint32_t g = static_cast<std::uint32_t>(r & 3u);
     half8v hi, lo;
     split8(v, s, hi, lo);
     // As a tree: a Q4_K product leans on this sum (offset times sum against
-    // codes times values), and its rounding is common to every output.
-    float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-    sum *= s;
+    // codes times values), and its rounding is common to every output.  Of the
+    // scaled values, which stay below 2^15: eight large floats would overflow.
+    const float sum01 = v[0] * s + v[1] * s, sum23 = v[2] * s + v[3] * s;
+    const float sum45 = v[4] * s + v[5] * s, sum67 = v[6] * s + v[7] * s;
+    float sum = (sum01 + sum23) + (sum45 + sum67);
     sum += __shfl_xor(sum, 1);
     sum += __shfl_xor(sum, 2);
     const std::uint32_t lane = (m & 15u) + 16u * g;

@@ -110,6 +110,35 @@ def test_stream_outliers_keep_small_channels(torch_cuda, hip_ctx):
         mat.release()
 
 
+@pytest.mark.parametrize("k,n,m,path,wsplit", [(2048, 20000, 20, 0, 0), (2048, 640, 24, 2, 0), (2048, 640, 40, 0, 1)],
+                         ids=["stream", "skinny", "wsplit"])
+def test_q4_k_block_sums_of_large_values(torch_cuda, hip_ctx, k, n, m, path, wsplit):
+    """Runs of eight neighbours near 1e38: their sum is past f32's range, the
+    scaled one is not, and neither is any output."""
+    torch = torch_cuda
+    canon = helpers.weights(capi.TYPE_Q4_K, k, n, seed=8)
+    mat = capi.Matrix(hip_ctx, capi.TYPE_Q4_K, k, n, canon, canon.nbytes, on_device=False)
+    try:
+        hip_ctx.set_decode_path(path, 0, 0)
+        hip_ctx.set_wsplit(wsplit, 0, 0, 0, 0, 1 if wsplit else 0)
+        x = helpers.activations(m, k, seed=9)
+        x[1, 64:72] = 1e38
+        x[m - 1, 1000:1016] = -9e37
+        rows = np.arange(0, n, max(1, n // 200)).astype(np.uint64)
+        y = torch.empty((m, n), dtype=torch.float32, device="cuda:0")
+        mat.linear(torch.from_numpy(x).to("cuda:0"), y, m)
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()
+        assert np.isfinite(got).all(), mat.plan(m)
+        want = oracle.linear_row_list(capi.TYPE_Q4_K, canon, k, n, x, rows)
+        for r in range(m):
+            assert helpers.rel_l2(got[r, rows.astype(np.int64)], want[r]) <= DECODE_TOL, (r, mat.plan(m))
+    finally:
+        hip_ctx.set_decode_path(0, 0, 0)
+        hip_ctx.set_wsplit(0, 0, 0, 0, 0, 0)
+        mat.release()
+
+
 # (format, K, N of the fused gate|up, widths): one and two tiles per wave,
 # eight waves, a last workgroup short of tiles, an odd count of gate tiles;
 # the Q8_0 rows at 2000..4096 row tiles and 17..32 rows sum their two K splits
