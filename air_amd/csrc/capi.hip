@@ -353,7 +353,7 @@ bool dense_prefill(const air_hip_context* ctx, const air_hip_matrix* m, std::uin
 
 // Which kernels a linear of `rows` rows runs on, decided in one place for
 // the launch path and for air_hip_linear_plan.
-enum class Route { prefill, gemv, fused, skinny_x, skinny_loaded, decode_linear, dense, wsplit };
+enum class Route { prefill, gemv, fused, skinny_x, skinny_loaded, decode_linear, dense, wsplit, stream };
 
 // No override of the 2..64-row decode kernels is set: each asks for a kernel
 // of its own, and the streaming kernel has none.
@@ -364,28 +364,15 @@ bool decode_automatic(const air_hip_context* ctx) {
            w.depth == 0u && w.k_splits == 0u && w.split_x == 0u;
 }
 
-// The plan of the kernels over split activations: the streaming kernel where
-// the automatic route prefers it, else a skinny kernel.
 SkinnyShape skinny_plan(const air_hip_context* ctx, const TilePlanes& p, std::uint32_t rows) {
-    if (decode_automatic(ctx) && stream_preferred(p, rows)) return plan_stream(p, rows);
     return plan_skinny(p, rows, ctx->skinny_tile_n, ctx->skinny_splits, ctx->skinny_lds_stages, ctx->skinny_waves);
 }
 
-// A dense F16 or Q6_K matrix at decode widths runs the streaming kernel on
-// its rows where the automatic route prefers it and what it needs fits the
-// no-allocation entry point's scratch (so both entry points take one route).
-bool dense_stream(const air_hip_context* ctx, const air_hip_matrix* m, std::uint32_t rows, int tactic) {
-    const DenseTuning& t = ctx->dense_tuning;
-    if (!m->dense || !m->gemm.codes || tactic == AIR_HIP_LINEAR_PREFILL || rows > AIR_HIP_MAX_DECODE_ROWS ||
-        t.path != 0u || t.shape.tile_n != 0u || t.shape.waves != 0u || t.shape.depth != 0u ||
-        (m->dense_storage != kF16 && m->dense_storage != kQ6_K) || !decode_automatic(ctx) ||
-        !stream_preferred(m->gemm, rows)) {
-        return false;
-    }
-    const SkinnyShape s = plan_stream(m->gemm, rows);
-    const std::uint64_t kp = ceil_div(m->gemm.k, kSplitK) * kSplitK;
-    return ceil_div(split_workspace_bytes(kp, rows), 256u) * 256u + skinny_partials_bytes(s, rows, m->gemm.n) <=
-           kNoAllocScratchBytes;
+// The plan over activations a caller loaded: the streaming kernel where the
+// automatic route prefers it, else a skinny kernel.
+SkinnyShape loaded_plan(const air_hip_context* ctx, const TilePlanes& p, std::uint32_t rows) {
+    if (decode_automatic(ctx) && stream_preferred(p, rows)) return plan_stream(p, rows);
+    return skinny_plan(ctx, p, rows);
 }
 
 // The skinny kernel straight from the f32 rows, or over activations split
@@ -396,7 +383,6 @@ bool dense_stream(const air_hip_context* ctx, const air_hip_matrix* m, std::uint
 // M = 64.  Q4_K with four activation tiles would also spill in it.
 Route skinny_route(const air_hip_context* ctx, const air_hip_matrix* m, std::uint32_t rows) {
     const SkinnyShape shape = skinny_plan(ctx, m->planes, rows);
-    if (shape.stream) return Route::skinny_loaded;
     // From 17 rows the split activations feed the LDS pipeline, which beats
     // the f32-input kernel on the narrow 7B matrices too, split launch
     // included (Q8_0, M = 32: q|k|v 18.4 -> 16.2 us, o 16.3 -> 14.7, down
@@ -407,14 +393,14 @@ Route skinny_route(const air_hip_context* ctx, const air_hip_matrix* m, std::uin
     return (!narrow || (m->planes.type == kQ4_K && shape.mt == 4u)) ? Route::skinny_loaded : Route::skinny_x;
 }
 
-// tactic is already validated; rows >= 1.
-Route route_linear(const air_hip_context* ctx, const air_hip_matrix* m, std::uint32_t rows, int tactic) {
+// The route without the streaming kernel.  tactic is already validated;
+// rows >= 1.
+Route base_route(const air_hip_context* ctx, const air_hip_matrix* m, std::uint32_t rows, int tactic) {
     if (m->dense) return Route::dense;   // every tactic and width
     if (tactic == AIR_HIP_LINEAR_PREFILL || (tactic == AIR_HIP_LINEAR_AUTO && rows > AIR_HIP_MAX_DECODE_ROWS)) {
         return Route::prefill;
     }
     if (rows == 1u) return Route::gemv;
-    if (decode_automatic(ctx) && stream_preferred(m->planes, rows)) return Route::skinny_loaded;
     if (rows <= AIR_HIP_MAX_DECODE_ROWS &&
         (ctx->wsplit_mode == 1u ||
          (ctx->wsplit_mode == 0u && ctx->decode_path == 0u && wsplit_preferred(m->planes, rows)))) {
@@ -437,18 +423,100 @@ Route route_linear(const air_hip_context* ctx, const air_hip_matrix* m, std::uin
     return Route::decode_linear;
 }
 
-// The streaming decode linear over `planes` (the matrix's tiles or dense
-// rows).  Its activations are the split an epilogue just left for these rows
+// Scratch a decode route needs in the no-allocation entry point: the split
+// activations, then the K-split partials.
+struct RouteScratch {
+    std::uint64_t ws{0};
+    std::uint64_t partials{0};
+    std::uint64_t total() const { return ws + partials; }
+};
+RouteScratch route_scratch(const air_hip_context* ctx, const air_hip_matrix* m, std::uint32_t rows, Route route) {
+    const TilePlanes& p = m->dense ? m->gemm : m->planes;
+    const std::uint64_t split =
+        ceil_div(split_workspace_bytes(ceil_div(p.k, kSplitK) * kSplitK, rows), 256u) * 256u;
+    RouteScratch s;
+    switch (route) {
+    case Route::stream:
+        s.ws = split;
+        s.partials = skinny_partials_bytes(plan_stream(p, rows), rows, p.n);
+        break;
+    case Route::skinny_x:
+    case Route::skinny_loaded:
+        s.ws = route == Route::skinny_loaded ? split : 0u;
+        s.partials = skinny_partials_bytes(skinny_plan(ctx, p, rows), rows, p.n);
+        break;
+    case Route::wsplit: {
+        const WsplitShape w = plan_wsplit(p, rows, ctx->wsplit_tuning);
+        s.ws = w.split_x ? split : 0u;
+        s.partials = wsplit_partials_bytes(w, rows, p.n);
+        break;
+    }
+    case Route::decode_linear: s.ws = split; break;
+    default: break;
+    }
+    return s;
+}
+
+// Whether the automatic route takes the streaming kernel, over a matrix's
+// tiles or its dense F16 or Q6_K rows.  Not where only the route without it
+// fits the no-allocation entry point's scratch: both entry points take one
+// route, and what that one accepted it accepts.
+bool stream_route(const air_hip_context* ctx, const air_hip_matrix* m, std::uint32_t rows, int tactic) {
+    if (rows < 2u || rows > AIR_HIP_MAX_DECODE_ROWS || tactic == AIR_HIP_LINEAR_PREFILL || !decode_automatic(ctx)) {
+        return false;
+    }
+    if (m->dense) {
+        const DenseTuning& t = ctx->dense_tuning;
+        if (!m->gemm.codes || t.path != 0u || t.shape.tile_n != 0u || t.shape.waves != 0u || t.shape.depth != 0u ||
+            (m->dense_storage != kF16 && m->dense_storage != kQ6_K)) {
+            return false;
+        }
+    }
+    if (!stream_preferred(m->dense ? m->gemm : m->planes, rows)) return false;
+    return route_scratch(ctx, m, rows, Route::stream).total() <= kNoAllocScratchBytes ||
+           route_scratch(ctx, m, rows, base_route(ctx, m, rows, tactic)).total() > kNoAllocScratchBytes;
+}
+
+Route route_linear(const air_hip_context* ctx, const air_hip_matrix* m, std::uint32_t rows, int tactic) {
+    return stream_route(ctx, m, rows, tactic) ? Route::stream : base_route(ctx, m, rows, tactic);
+}
+
+bool capturing(const air_hip_context* ctx) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
+}
+
+// Whether the epilogue of the call before left the row-scaled split of
+// exactly these rows (`ready`: the source it recorded) in the workspace.
+bool split_ready(const air_hip_context* ctx, const TilePlanes& p, const float* x, std::uint32_t rows,
+                 const void* ready) {
+    return ready == x && ctx->loaded_k == p.k && ctx->loaded_rows == rows && ctx->loaded_row_scaled;
+}
+
+// Whether a streaming launch has its buffers, or may grow them: not while the
+// stream is captured, where the linear takes the route without it instead
+// (which on dense rows, and on tiles read straight from the f32 rows, needs
+// none).
+bool stream_room(const air_hip_context* ctx, const TilePlanes& p, std::uint32_t rows, std::uint64_t partial_bytes,
+                 bool ready) {
+    const std::uint64_t kp = ceil_div(p.k, kSplitK) * kSplitK;
+    return ((ready || split_workspace_bytes(kp, rows) <= ctx->stream_rows_bytes) &&
+            partial_bytes <= ctx->split_partials_bytes) ||
+           !capturing(ctx);
+}
+
+// The streaming decode linear (plan `shape`) over the matrix's tiles or dense
+// rows.  Its activations are the split an epilogue just left for these rows
 // (`ready`), or are split into a buffer of its own: activations a caller
 // loaded stay as they are.
-int run_stream(air_hip_context* ctx, const air_hip_matrix* m, const TilePlanes& planes, const float* x, float* y,
+int run_stream(air_hip_context* ctx, const air_hip_matrix* m, const SkinnyShape& shape, const float* x, float* y,
                const float* bias, std::uint32_t rows, const SplitEpilogue* epilogue, bool* applied, const void* ready) {
-    const SkinnyShape shape = skinny_plan(ctx, planes, rows);
+    const TilePlanes& planes = m->dense ? m->gemm : m->planes;
     SkinnyShape swiglu{};
     const bool fused = epilogue && epilogue->kind == kEpilogueSwiglu && plan_stream_swiglu(planes, rows, shape, swiglu);
     const std::uint64_t kp = ceil_div(planes.k, kSplitK) * kSplitK;
     SplitWorkspace ws{};
-    if (ready == x && ctx->loaded_k == planes.k && ctx->loaded_rows == rows && ctx->loaded_row_scaled) {
+    if (split_ready(ctx, planes, x, rows, ready)) {
         ws = carve_split_workspace(ctx->workspace, kp, rows);
     } else {
         const int rc = grow_buffer(ctx, &ctx->stream_rows, &ctx->stream_rows_bytes, split_workspace_bytes(kp, rows),
@@ -486,11 +554,12 @@ int run_stream(air_hip_context* ctx, const air_hip_matrix* m, const TilePlanes& 
 int run_skinny_x(air_hip_context* ctx, const air_hip_matrix* m, const float* x, float* y, const float* bias,
                  std::uint32_t rows, const SplitEpilogue* epilogue, bool* applied, const void* ready) {
     const SkinnyShape shape = skinny_plan(ctx, m->planes, rows);
-    // The streaming kernel, or a SwiGLU it takes off the eight-wave kernel's hands.
+    // A SwiGLU the streaming kernel takes off the eight-wave kernel's hands.
     SkinnyShape swiglu{};
-    if (shape.stream || (decode_automatic(ctx) && epilogue && epilogue->kind == kEpilogueSwiglu &&
-                         plan_stream_swiglu(m->planes, rows, shape, swiglu))) {
-        return run_stream(ctx, m, m->planes, x, y, bias, rows, epilogue, applied, ready);
+    if (decode_automatic(ctx) && epilogue && epilogue->kind == kEpilogueSwiglu &&
+        plan_stream_swiglu(m->planes, rows, shape, swiglu) &&
+        stream_room(ctx, m->planes, rows, 0u, split_ready(ctx, m->planes, x, rows, ready))) {
+        return run_stream(ctx, m, shape, x, y, bias, rows, epilogue, applied, ready);
     }
     if (skinny_route(ctx, m, rows) == Route::skinny_loaded) {
         int rc = load_activations_for(ctx, x, m->planes.k, rows, ready);
@@ -570,10 +639,7 @@ std::uint64_t* chain_for(air_hip_context* ctx, std::uint32_t splits, std::uint32
     if (ctx->chain_mode == 0u && !chain_auto(splits, m, n, stream)) return nullptr;
     const std::uint64_t bytes = chain_slot_bytes(splits, m, n);
     if (bytes <= ctx->chain_slots_bytes) return ctx->chain_slots;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
-        return nullptr;
-    }
+    if (capturing(ctx)) return nullptr;
     const std::uint64_t grown = std::max<std::uint64_t>(bytes, ctx->chain_slots_bytes + ctx->chain_slots_bytes / 2);
     void* p = nullptr;
     if (hipMalloc(&p, grown) != hipSuccess) return nullptr;
@@ -837,6 +903,10 @@ int air_hip_context_reserve(air_hip_context* ctx, uint64_t max_k, uint32_t max_m
         rc = grow_buffer(ctx, &ctx->stream_rows, &ctx->stream_rows_bytes,
                          split_workspace_bytes(kp, std::min<std::uint32_t>(max_m, AIR_HIP_MAX_DECODE_ROWS)),
                          "stream activations");
+    }
+    // Its K splits fill at most one round of 256 workgroups of 128 outputs a row.
+    if (rc == AIR_HIP_OK && max_m > 1u) {
+        rc = ensure_split_buffers(ctx, 256ull * 128u * 4u * std::min<std::uint32_t>(max_m, AIR_HIP_MAX_DECODE_ROWS), 0u);
     }
     if (rc != AIR_HIP_OK || max_m <= kFusedMaxRows) return rc;
     PrefillShape unsplit{};
@@ -1271,7 +1341,7 @@ int linear_loaded(air_hip_context* ctx, const air_hip_matrix* m, float* y, const
         return fail(AIR_HIP_INVALID_STATE, "activations were loaded for another decode path; load them again");
     }
     if (skinny) {
-        const SkinnyShape shape = skinny_plan(ctx, m->planes, rows);
+        const SkinnyShape shape = loaded_plan(ctx, m->planes, rows);
         const std::uint64_t partial_bytes = skinny_partials_bytes(shape, rows, m->planes.n);
         if (partial_bytes > 0u) {
             const int rc = ensure_split_buffers(ctx, partial_bytes, 0u);
@@ -1309,7 +1379,19 @@ int linear_rows(air_hip_context* ctx, const air_hip_matrix* m, const float* x, f
     }
     if (m->owner->device != ctx->device) return fail(AIR_HIP_INVALID_ARGUMENT, "matrix belongs to another device");
     if (rows == 0) return fail(AIR_HIP_INVALID_ARGUMENT, "linear batch width must be non-zero");
-    const Route route = route_linear(ctx, m, rows, tactic);
+    Route route = route_linear(ctx, m, rows, tactic);
+    if (route == Route::stream) {
+        if (reinterpret_cast<std::uintptr_t>(x) % 16u != 0) return fail(AIR_HIP_INVALID_ARGUMENT, "x must be 16-byte aligned");
+        DeviceScope scope(ctx->device);
+        if (scope.status() != hipSuccess) return hip_fail(scope.status(), "hipSetDevice");
+        const TilePlanes& planes = m->dense ? m->gemm : m->planes;
+        const SkinnyShape shape = plan_stream(planes, rows);
+        if (stream_room(ctx, planes, rows, skinny_partials_bytes(shape, rows, planes.n),
+                        split_ready(ctx, planes, x, rows, ready))) {
+            return run_stream(ctx, m, shape, x, y, bias, rows, epilogue, applied, ready);
+        }
+        route = base_route(ctx, m, rows, tactic);
+    }
     if (route == Route::dense) {
         if (reinterpret_cast<std::uintptr_t>(x) % 16u != 0) return fail(AIR_HIP_INVALID_ARGUMENT, "x must be 16-byte aligned");
         DeviceScope scope(ctx->device);
@@ -1318,7 +1400,6 @@ int linear_rows(air_hip_context* ctx, const air_hip_matrix* m, const float* x, f
             return run_prefill(ctx, m, x, y, bias, rows, prefill_ready, ctx->prefill_source_k, ctx->prefill_source_rows,
                                epilogue, applied);
         }
-        if (dense_stream(ctx, m, rows, tactic)) return run_stream(ctx, m, m->gemm, x, y, bias, rows, epilogue, applied, ready);
         const hipError_t err = launch_dense_linear(m->dense, m->dense_storage, m->planes.k, m->planes.n, x, bias, y, rows,
                                                      ctx->stream, ctx->dense_tuning);
         if (err != hipSuccess) return hip_fail(err, "dense_rows_kernel / dense_gemm_kernel");
@@ -1384,6 +1465,15 @@ std::string describe_linear(const air_hip_context* ctx, const air_hip_matrix* m,
                       : m->planes.type == kQ4_0 ? "q4_0" : "q4_k";
     char buf[256];
     switch (route_linear(ctx, m, rows, tactic)) {
+    case Route::stream: {
+        const SkinnyShape k = plan_stream(m->dense ? m->gemm : m->planes, rows);
+        const char* tail = split_tail(ctx, k.splits, rows, m->planes.n, true);
+        std::snprintf(buf, sizeof buf, "split_rows_kernel + stream_kernel<%s> mt=%u tile_n=%u waves=%u+2 groups=%u "
+                      "splits=%u%s%s", m->type == kQ6_K ? "q6_k" : m->type == kF16 ? "f16" : fmt, k.mt, k.tile_n,
+                      k.waves, k.groups, k.splits, tail,
+                      m->type == kQ6_K ? " (dense q6_k super-block rows)" : m->type == kF16 ? " (dense f16 rows)" : "");
+        break;
+    }
     case Route::dense: {
         const char* t = m->type == kF32 ? "f32" : m->type == kF16 ? "f16" : m->type == kBF16 ? "bf16" : "q6_k";
         if (dense_prefill(ctx, m, rows, tactic)) {
@@ -1403,14 +1493,6 @@ std::string describe_linear(const air_hip_context* ctx, const air_hip_matrix* m,
             const Q6kGemvPlan g = plan_q6k_gemv(m->planes.k, m->planes.n, ctx->dense_tuning.shape);
             std::snprintf(buf, sizeof buf, "q6k_gemv_kernel waves=%u units=%u depth=%u (dense q6_k super-block rows)",
                           g.waves, g.units, g.depth);
-            break;
-        }
-        if (dense_stream(ctx, m, rows, tactic)) {
-            const SkinnyShape k = plan_stream(m->gemm, rows);
-            std::snprintf(buf, sizeof buf, "split_rows_kernel + stream_kernel<%s> mt=%u tile_n=%u waves=%u+2 groups=%u "
-                          "splits=%u%s (dense %s %s)", t, k.mt, k.tile_n, k.waves, k.groups, k.splits,
-                          split_tail(ctx, k.splits, rows, m->planes.n, true), t,
-                          m->type == kQ6_K ? "super-block rows" : "rows");
             break;
         }
         if (dense_mfma_route(m->dense_storage, m->planes.k, m->planes.n, rows, ctx->dense_tuning)) {
@@ -1463,12 +1545,6 @@ std::string describe_linear(const air_hip_context* ctx, const air_hip_matrix* m,
     case Route::skinny_loaded: {
         const bool loaded = route_linear(ctx, m, rows, tactic) == Route::skinny_loaded;
         const SkinnyShape k = skinny_plan(ctx, m->planes, rows);
-        if (k.stream) {
-            std::snprintf(buf, sizeof buf, "split_rows_kernel + stream_kernel<%s> mt=%u tile_n=%u waves=%u+2 groups=%u "
-                          "splits=%u%s", fmt, k.mt, k.tile_n, k.waves, k.groups, k.splits,
-                          split_tail(ctx, k.splits, rows, m->planes.n, true));
-            break;
-        }
         const bool lds = loaded && k.lds_stages >= 2u;
         char stages[32] = "";
         if (lds) std::snprintf(stages, sizeof stages, " lds_stages=%u%s", k.lds_stages, k.waves == 8u ? " waves=8" : "");
@@ -1520,22 +1596,15 @@ int air_hip_linear_noalloc(air_hip_context* ctx, const air_hip_matrix* m, const 
     }
     if (m->owner->device != ctx->device) return fail(AIR_HIP_INVALID_ARGUMENT, "matrix belongs to another device");
     if (reinterpret_cast<std::uintptr_t>(x) % 16u != 0) return fail(AIR_HIP_INVALID_ARGUMENT, "x must be 16-byte aligned");
-    if (m->dense) {   // the same launches as air_hip_linear
+    // Same route, plans and kernels as air_hip_linear with this context's
+    // settings, so the results are bit-identical; only the buffers differ:
+    // the split activations at the start of the scratch array, the K-split
+    // partials after them (256-byte aligned).  Each launch writes every
+    // scratch byte it later reads, so nothing needs clearing between calls.
+    const Route route = route_linear(ctx, m, rows, tactic);
+    if (route == Route::dense || (m->dense && !ctx->noalloc_scratch)) {   // no scratch: air_hip_linear's launch
         DeviceScope scope(ctx->device);
         if (scope.status() != hipSuccess) return hip_fail(scope.status(), "hipSetDevice");
-        if (ctx->noalloc_scratch && dense_stream(ctx, m, rows, tactic)) {
-            const SkinnyShape shape = plan_stream(m->gemm, rows);
-            const std::uint64_t kp = ceil_div(m->gemm.k, kSplitK) * kSplitK;
-            auto* base = static_cast<unsigned char*>(ctx->noalloc_scratch);
-            const SplitWorkspace ws = carve_split_workspace(base, kp, rows);
-            float* partials = reinterpret_cast<float*>(base + ceil_div(split_workspace_bytes(kp, rows), 256u) * 256u);
-            hipError_t err = launch_split_activations_rows(x, rows, m->gemm.k, kp, ws, ctx->stream);
-            if (err == hipSuccess) err = launch_stream_linear(m->gemm, ws, bias, y, rows, shape, partials, ctx->stream);
-            if (err != hipSuccess) return hip_fail(err, "stream_kernel");
-            ctx->decode_linear_calls.fetch_add(1, std::memory_order_relaxed);
-            ctx->decode_rows.fetch_add(rows, std::memory_order_relaxed);
-            return AIR_HIP_OK;
-        }
         const hipError_t err = launch_dense_linear(m->dense, m->dense_storage, m->planes.k, m->planes.n, x, bias, y, rows,
                                                      ctx->stream, ctx->dense_tuning);
         if (err != hipSuccess) return hip_fail(err, "dense_rows_kernel / dense_gemm_kernel");
@@ -1544,41 +1613,22 @@ int air_hip_linear_noalloc(air_hip_context* ctx, const air_hip_matrix* m, const 
         return AIR_HIP_OK;
     }
     if (!ctx->noalloc_scratch) return fail(AIR_HIP_INTERNAL_ERROR, "the device scratch array is not mapped");
-    // Same route, plans and kernels as air_hip_linear with this context's
-    // settings, so the results are bit-identical; only the buffers differ:
-    // the split activations at the start of the scratch array, the K-split
-    // partials after them (256-byte aligned).  Each launch writes every
-    // scratch byte it later reads, so nothing needs clearing between calls.
-    const Route route = route_linear(ctx, m, rows, tactic);
-    const TilePlanes& p = m->planes;
+    const TilePlanes& p = m->dense ? m->gemm : m->planes;
     const std::uint64_t kp = ceil_div(p.k, kSplitK) * kSplitK;
-    std::uint64_t ws_bytes = 0, partial_bytes = 0;
-    SkinnyShape shape{};
-    WsplitShape wshape{};
-    if (route == Route::skinny_x || route == Route::skinny_loaded) {
-        shape = skinny_plan(ctx, p, rows);
-        partial_bytes = skinny_partials_bytes(shape, rows, p.n);
-    }
-    if (route == Route::wsplit) {
-        wshape = plan_wsplit(p, rows, ctx->wsplit_tuning);
-        partial_bytes = wsplit_partials_bytes(wshape, rows, p.n);
-    }
-    if (route == Route::skinny_loaded || route == Route::decode_linear || (route == Route::wsplit && wshape.split_x)) {
-        ws_bytes = ceil_div(split_workspace_bytes(kp, rows), 256u) * 256u;
-    }
+    const RouteScratch need = route_scratch(ctx, m, rows, route);
     if (route == Route::fused && plan_decode_fused(p, rows, ctx->tuning).k_splits > 1u) {
         return fail(AIR_HIP_UNSUPPORTED, "the no-allocation linear does not run the fused kernel's cross-workgroup "
                     "K split (a context tuning override)");
     }
-    if (ws_bytes + partial_bytes > kNoAllocScratchBytes) {
+    if (need.total() > kNoAllocScratchBytes) {
         return fail(AIR_HIP_UNSUPPORTED, "this linear needs %llu bytes of scratch; the no-allocation array holds %llu",
-                    static_cast<unsigned long long>(ws_bytes + partial_bytes),
+                    static_cast<unsigned long long>(need.total()),
                     static_cast<unsigned long long>(kNoAllocScratchBytes));
     }
     DeviceScope scope(ctx->device);
     if (scope.status() != hipSuccess) return hip_fail(scope.status(), "hipSetDevice");
     auto* base = static_cast<unsigned char*>(ctx->noalloc_scratch);
-    float* partials = reinterpret_cast<float*>(base + ws_bytes);
+    float* partials = reinterpret_cast<float*>(base + need.ws);
     const SplitWorkspace ws = carve_split_workspace(base, kp, rows);
     hipError_t err = hipSuccess;
     switch (route) {
@@ -1590,19 +1640,24 @@ int air_hip_linear_noalloc(air_hip_context* ctx, const air_hip_matrix* m, const 
                                   ctx->stream);
         break;
     case Route::skinny_x:
-        err = launch_skinny_linear_x(p, x, bias, y, rows, shape, partials, ctx->stream);
+        err = launch_skinny_linear_x(p, x, bias, y, rows, skinny_plan(ctx, p, rows), partials, ctx->stream);
         break;
     case Route::skinny_loaded:
+    case Route::stream: {
+        const SkinnyShape shape = route == Route::stream ? plan_stream(p, rows) : skinny_plan(ctx, p, rows);
         err = launch_split_activations_rows(x, rows, p.k, kp, ws, ctx->stream);
         if (err == hipSuccess) err = launch_skinny_linear(p, ws, bias, y, rows, shape, partials, ctx->stream);
         break;
-    case Route::wsplit:
+    }
+    case Route::wsplit: {
+        const WsplitShape wshape = plan_wsplit(p, rows, ctx->wsplit_tuning);
         if (wshape.split_x) err = launch_split_activations_rows(x, rows, p.k, kp, ws, ctx->stream);
         if (err == hipSuccess) {
             err = launch_wsplit_linear(p, x, wshape.split_x ? &ws : nullptr, bias, y, rows, wshape, partials,
                                        ctx->stream);
         }
         break;
+    }
     case Route::decode_linear:
         err = launch_split_activations(x, rows, p.k, kp, ws, ctx->stream);
         if (err == hipSuccess) err = launch_decode_linear(p, ws, bias, y, rows, ctx->tuning, ctx->stream);

@@ -155,7 +155,10 @@ int air_hip_context_set_stream(air_hip_context* ctx, void* stream);
  * rows never allocate on the hot path (workspace sizing,
  * cuda_backend.cu:1825-1869); the f32 partials of a K-split prefill GEMM,
  * which depend on the output width, are sized by the first call that needs
- * them.  Without it the first call that needs more space allocates. */
+ * them, and so are those of the skinny and wave-split kernels.  Without it
+ * the first call that needs more space allocates; while the stream is being
+ * captured a linear at 2..64 rows whose streaming buffers are not there yet
+ * takes the kernel it would have without the streaming one. */
 int air_hip_context_reserve(air_hip_context* ctx, uint64_t max_k, uint32_t max_m);
 /* Counters and buffer sizes of the context (air_hip_stats above; no
  * counterpart in the reference). */

@@ -188,3 +188,55 @@ def test_stream_swiglu_bits(torch_cuda, hip_ctx, type_id, k, n, ms):
                 assert bool((got[m] == -7.0).all()), case
     finally:
         mat.release()
+
+
+@pytest.mark.parametrize("type_id,k,n,m", [(capi.TYPE_Q6_K, 8448, 1530, 13), (capi.TYPE_F16, 3104, 4200, 33),
+                                           (capi.TYPE_Q8_0, 2048, 16500, 5)])
+@pytest.mark.parametrize("reserved", [False, True], ids=["unreserved", "reserved"])
+def test_stream_first_call_under_capture(torch_cuda, reserved, type_id, k, n, m):
+    """A linear whose first call is recorded into a graph allocates nothing
+    there: without a reserve it takes the kernel it had before the streaming
+    one (no scratch), after one the streaming kernel, and replays repeat."""
+    torch = torch_cuda
+    dev = torch.device("cuda:0")
+    main = torch.cuda.current_stream(dev)
+    dense = type_id in (capi.TYPE_Q6_K, capi.TYPE_F16)
+    canon = (_weights if dense else helpers.weights)(type_id, k, n, seed=k + n)
+    ctx = capi.Context(0, main.cuda_stream)
+    mat = capi.Matrix(ctx, type_id, k, n, canon, canon.nbytes, on_device=False)
+    graph = torch.cuda.CUDAGraph()
+    try:
+        assert "stream_kernel" in mat.plan(m), mat.plan(m)
+        x = helpers.activations(m, k, seed=m + k)
+        xd = torch.from_numpy(x).to(dev)
+        y = torch.full((m, n), float("nan"), dtype=torch.float32, device=dev)
+        if reserved:
+            ctx.reserve(k, m)
+        generation = ctx.stats()["workspace_generation"]
+        capture = torch.cuda.Stream(dev)
+        ctx.set_stream(capture.cuda_stream)
+        with torch.cuda.graph(graph, stream=capture):
+            mat.linear(xd, y, m)
+        ctx.set_stream(main.cuda_stream)
+        assert ctx.stats()["workspace_generation"] == generation
+        eager = torch.empty((m, n), dtype=torch.float32, device=dev)
+        mat.linear_noalloc(xd, eager, m)          # the streaming kernel's bits
+        rows = np.arange(0, n, max(1, n // 200)).astype(np.uint64)
+        want = oracle.linear_row_list(type_id, canon, k, n, x, rows)
+        first = None
+        for _ in range(3):
+            y.fill_(float("nan"))
+            graph.replay()
+            mat.linear(xd, torch.empty((m, n), dtype=torch.float32, device=dev), m)   # eager work between
+            torch.cuda.synchronize()
+            got = y.cpu().numpy()
+            first = got if first is None else first
+            assert np.array_equal(got.view(np.uint32), first.view(np.uint32))
+            if reserved:
+                assert np.array_equal(got.view(np.uint32), eager.cpu().numpy().view(np.uint32))
+            assert helpers.rel_l2(got[:, rows.astype(np.int64)], want) <= (DENSE_TOL if dense else DECODE_TOL)
+    finally:
+        torch.cuda.synchronize()
+        graph = None
+        mat.release()
+        ctx.close()
