@@ -250,6 +250,7 @@ struct SkinnyShape {
     std::uint32_t lds_stages{0};  // Q8_0 from split activations: stages of the LDS pipeline (0 = registers)
     std::uint32_t waves{4};       // waves per workgroup: 4, or 8 on the LDS pipeline
     bool stream{false};           // the streaming kernel (linear_stream.hip): waves 8 or 10
+    bool block_scaled{false};     // over launch_split_activations_blocks' split, not the row-scaled one
 };
 // lds_stages: 0 automatic, 1 the register pipeline, 2..4 the LDS ring
 // (Q8_0 from split activations; other formats and f32 inputs ignore it).
@@ -266,9 +267,14 @@ std::uint64_t skinny_partials_bytes(const SkinnyShape& shape, std::uint32_t m, s
 hipError_t launch_skinny_linear(const TilePlanes& planes, const SplitWorkspace& ws, const float* bias, float* y,
                                 std::uint32_t m, const SkinnyShape& shape, float* partials, hipStream_t stream,
                                 const SplitEpilogue* epilogue = nullptr, std::uint64_t* chain = nullptr);
-// The streaming kernel (linear_stream.hip) over the same split activations:
-// whether the automatic route takes it for m rows, its plan (shape.stream), and
-// the launch (launch_skinny_linear calls it for such a shape).
+// The row-scaled split's layout with one scale per (row, 32-block):
+// inv_scale[b][m], block sums of the values so scaled (M <= 64).
+hipError_t launch_split_activations_blocks(const float* x, std::uint32_t m, std::uint64_t k, std::uint64_t kp,
+                                           const SplitWorkspace& ws, hipStream_t stream);
+// The streaming kernel (linear_stream.hip) over either split: whether the
+// automatic route takes it for m rows, its plan (shape.stream; block_scaled is
+// the caller's to set, and always set over dense rows), and the launch
+// (launch_skinny_linear calls it for such a shape).
 bool stream_preferred(const TilePlanes& planes, std::uint32_t m);
 SkinnyShape plan_stream(const TilePlanes& planes, std::uint32_t m);
 hipError_t launch_stream_linear(const TilePlanes& planes, const SplitWorkspace& ws, const float* bias, float* y,

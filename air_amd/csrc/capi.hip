@@ -481,6 +481,23 @@ Route route_linear(const air_hip_context* ctx, const air_hip_matrix* m, std::uin
     return stream_route(ctx, m, rows, tactic) ? Route::stream : base_route(ctx, m, rows, tactic);
 }
 
+// The streaming plan of route_linear's choice.  It holds the activations in no
+// fewer bits than the route it stands in for: one scale per (row, 32-block),
+// but for the routes over the row-scaled split.
+SkinnyShape stream_plan(const air_hip_context* ctx, const air_hip_matrix* m, std::uint32_t rows, int tactic) {
+    SkinnyShape s = plan_stream(m->dense ? m->gemm : m->planes, rows);
+    const Route base = base_route(ctx, m, rows, tactic);
+    s.block_scaled = !(base == Route::skinny_loaded ||
+                       (base == Route::wsplit && plan_wsplit(m->planes, rows, ctx->wsplit_tuning).split_x));
+    return s;
+}
+
+hipError_t split_for_stream(const SkinnyShape& s, const float* x, std::uint32_t rows, std::uint64_t k, std::uint64_t kp,
+                            const SplitWorkspace& ws, hipStream_t stream) {
+    return s.block_scaled ? launch_split_activations_blocks(x, rows, k, kp, ws, stream)
+                          : launch_split_activations_rows(x, rows, k, kp, ws, stream);
+}
+
 bool capturing(const air_hip_context* ctx) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
@@ -516,15 +533,15 @@ int run_stream(air_hip_context* ctx, const air_hip_matrix* m, const SkinnyShape&
     const bool fused = epilogue && epilogue->kind == kEpilogueSwiglu && plan_stream_swiglu(planes, rows, shape, swiglu);
     const std::uint64_t kp = ceil_div(planes.k, kSplitK) * kSplitK;
     SplitWorkspace ws{};
-    if (split_ready(ctx, planes, x, rows, ready)) {
+    if (!shape.block_scaled && split_ready(ctx, planes, x, rows, ready)) {
         ws = carve_split_workspace(ctx->workspace, kp, rows);
     } else {
         const int rc = grow_buffer(ctx, &ctx->stream_rows, &ctx->stream_rows_bytes, split_workspace_bytes(kp, rows),
                                    "stream activations");
         if (rc != AIR_HIP_OK) return rc;
         ws = carve_split_workspace(ctx->stream_rows, kp, rows);
-        const hipError_t err = launch_split_activations_rows(x, rows, planes.k, kp, ws, ctx->stream);
-        if (err != hipSuccess) return hip_fail(err, "split_rows_kernel");
+        const hipError_t err = split_for_stream(shape, x, rows, planes.k, kp, ws, ctx->stream);
+        if (err != hipSuccess) return hip_fail(err, shape.block_scaled ? "split_blocks_kernel" : "split_rows_kernel");
     }
     if (fused) {
         const hipError_t err = launch_stream_swiglu(planes, ws, bias, epilogue->out, rows, swiglu, ctx->stream);
@@ -1385,9 +1402,9 @@ int linear_rows(air_hip_context* ctx, const air_hip_matrix* m, const float* x, f
         DeviceScope scope(ctx->device);
         if (scope.status() != hipSuccess) return hip_fail(scope.status(), "hipSetDevice");
         const TilePlanes& planes = m->dense ? m->gemm : m->planes;
-        const SkinnyShape shape = plan_stream(planes, rows);
+        const SkinnyShape shape = stream_plan(ctx, m, rows, tactic);
         if (stream_room(ctx, planes, rows, skinny_partials_bytes(shape, rows, planes.n),
-                        split_ready(ctx, planes, x, rows, ready))) {
+                        !shape.block_scaled && split_ready(ctx, planes, x, rows, ready))) {
             return run_stream(ctx, m, shape, x, y, bias, rows, epilogue, applied, ready);
         }
         route = base_route(ctx, m, rows, tactic);
@@ -1466,10 +1483,10 @@ std::string describe_linear(const air_hip_context* ctx, const air_hip_matrix* m,
     char buf[256];
     switch (route_linear(ctx, m, rows, tactic)) {
     case Route::stream: {
-        const SkinnyShape k = plan_stream(m->dense ? m->gemm : m->planes, rows);
+        const SkinnyShape k = stream_plan(ctx, m, rows, tactic);
         const char* tail = split_tail(ctx, k.splits, rows, m->planes.n, true);
-        std::snprintf(buf, sizeof buf, "split_rows_kernel + stream_kernel<%s> mt=%u tile_n=%u waves=%u+2 groups=%u "
-                      "splits=%u%s%s", m->type == kQ6_K ? "q6_k" : m->type == kF16 ? "f16" : fmt, k.mt, k.tile_n,
+        std::snprintf(buf, sizeof buf, "%s + stream_kernel<%s> mt=%u tile_n=%u waves=%u+2 groups=%u "
+                      "splits=%u%s%s", k.block_scaled ? "split_blocks_kernel" : "split_rows_kernel", m->type == kQ6_K ? "q6_k" : m->type == kF16 ? "f16" : fmt, k.mt, k.tile_n,
                       k.waves, k.groups, k.splits, tail,
                       m->type == kQ6_K ? " (dense q6_k super-block rows)" : m->type == kF16 ? " (dense f16 rows)" : "");
         break;
@@ -1644,8 +1661,8 @@ int air_hip_linear_noalloc(air_hip_context* ctx, const air_hip_matrix* m, const 
         break;
     case Route::skinny_loaded:
     case Route::stream: {
-        const SkinnyShape shape = route == Route::stream ? plan_stream(p, rows) : skinny_plan(ctx, p, rows);
-        err = launch_split_activations_rows(x, rows, p.k, kp, ws, ctx->stream);
+        const SkinnyShape shape = route == Route::stream ? stream_plan(ctx, m, rows, tactic) : skinny_plan(ctx, p, rows);
+        err = split_for_stream(shape, x, rows, p.k, kp, ws, ctx->stream);
         if (err == hipSuccess) err = launch_skinny_linear(p, ws, bias, y, rows, shape, partials, ctx->stream);
         break;
     }

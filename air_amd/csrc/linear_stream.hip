@@ -22,6 +22,9 @@
 //     rows and 28 at 64 (7B, Q8_0, timed with the staging left out);
 //   * one bare barrier per chunk; a chunk's fragments are read from LDS one
 //     stage ahead of the MFMAs that use them;
+//   * the activations come split under one power-of-two scale per row, or per
+//     (row, 32-block) where the kernel this one is taken instead of scaled
+//     blocks or steps (BLOCKS);
 //   * the K sum is formed in levels where registers allow (kLevels): pairs
 //     of steps, trips of the ring, then the total.  One running sum of the
 //     112 blocks of K = 3584 is 2.3e-7 from 64 bits (relative L2, Q8_0), the
@@ -77,7 +80,7 @@ struct StreamArgs {
     std::uint64_t n, k;
     const u32x4* xs;             // split activations [block][MT][2][64] x 16 B
     std::uint32_t blocks;        // 32-element blocks of the workspace
-    const float* inv_scale;      // [mp] inverse power-of-two scale of each row
+    const float* inv_scale;      // [mp] inverse power-of-two scale of each row; BLOCKS: [block][mp]
     const float* block_sums;     // [block][mp] sums of the scaled values (Q4_K)
     const float* bias;           // fused when not split over workgroups
     float* out;                  // y, or partials [splits][m][n]
@@ -260,8 +263,9 @@ constexpr unsigned kRing = FMT == kQ8_0 || FMT == kF16 ? (MT <= 2 ? 8u : 4u) / T
 constexpr int kProducers = 2;
 // Levels of the K sum: three, or as many as leave no register in scratch.
 template <int FMT, int MT, int TN>
-constexpr unsigned kLevels = FMT == kF16 && MT == 2 && TN == 2 ? 2u
-                             : MT <= 2 || FMT == kQ6_K         ? 3u
+constexpr unsigned kLevels = FMT == kF16 && MT == 2 && TN == 2              ? 2u
+                             : FMT == kQ6_K && (MT >= 3 || (MT == 2 && TN == 2)) ? 2u
+                             : MT <= 2                                         ? 3u
                              : FMT == kQ4_K || (MT == 4 && TN == 2) ? 1u
                                                                     : 2u;
 
@@ -275,8 +279,15 @@ constexpr unsigned kLevels = FMT == kF16 && MT == 2 && TN == 2 ? 2u
 // SERIAL: the K splits of a plan that sums them in a reduction, one after the
 // other in one workgroup: each in one running sum, scaled, then added from
 // zero in split order -- that plan's bits.
-template <int FMT, int MT, int TN, int W, bool SWIGLU, bool SERIAL>
+// BLOCKS: the activations were split under one scale per (row, 32-block), which
+// travels with the fragments and is undone on each block's products; else under
+// one per row, undone on the total.  Where the kernel that would otherwise run
+// scales steps or blocks, the rows' small blocks beside a large one keep their
+// bits only so.
+template <int FMT, int MT, int TN, int W, bool SWIGLU, bool SERIAL, bool BLOCKS>
 __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) void stream_kernel(StreamArgs a) {
+    static_assert(!(SERIAL && BLOCKS), "the serial plan scales rows");
+    static_assert(BLOCKS || !dense_storage(FMT), "dense rows take block scales");
     constexpr unsigned P = kProducers;
     constexpr unsigned U = kUnit<FMT>;
     constexpr unsigned D = kRing<FMT, MT, TN>;
@@ -295,8 +306,11 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
     constexpr unsigned kFrags = 2u * C * 2u * MT;           // 1 KiB activation fragments per chunk
     constexpr unsigned kXBytes = kFrags * 1024u;
     constexpr unsigned kSumLoads = kSums ? 2u * C * kMp / 64u : 0u;   // 64-float loads of a chunk's block sums
-    constexpr unsigned kChunkBytes = kXBytes + kSumLoads * 256u;
-    constexpr unsigned kXLoads = (kFrags + P - 1u) / P + (kSumLoads + P - 1u) / P;   // per producer and chunk
+    constexpr unsigned kInvLoads = BLOCKS ? 2u * C * kMp / 64u : 0u;  // and of its inverse scales
+    constexpr unsigned kInvAt = kXBytes + kSumLoads * 256u;
+    constexpr unsigned kChunkBytes = kInvAt + kInvLoads * 256u;
+    constexpr unsigned kXLoads =                            // per producer and chunk
+        (kFrags + P - 1u) / P + (kSumLoads + P - 1u) / P + (kInvLoads + P - 1u) / P;
     static_assert(kBody % C == 0u && kBody % (D * U) == 0u, "a trip is whole chunks and ring turns");
     static_assert((kBuffers - 2u) * kXLoads < 64u, "vmcnt is six bits");
     __shared__ __attribute__((aligned(1024))) unsigned char chunks[kBuffers * kChunkBytes];
@@ -330,13 +344,17 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
                 const std::uint32_t b = min(b0 + f / (2u * MT), a.blocks - 1u);
                 lds_load16(a.xs + (static_cast<std::uint64_t>(b) * (2u * MT) + f % (2u * MT)) * 64u + lane, base + f * 1024u);
             }
+            const auto per_block = [&](const float* from, unsigned loads, unsigned at) __attribute__((always_inline)) {
 #pragma unroll
-            for (unsigned j = 0; j < (kSumLoads + P - 1u) / P; ++j) {
-                const unsigned q = min(producer + P * j, kSumLoads - 1u);
-                const unsigned e = q * 64u + lane;
-                const std::uint32_t b = min(b0 + e / kMp, a.blocks - 1u);
-                lds_load4(a.block_sums + static_cast<std::uint64_t>(b) * kMp + e % kMp, base + kXBytes + q * 256u);
-            }
+                for (unsigned j = 0; j < (loads + P - 1u) / P; ++j) {
+                    const unsigned q = min(producer + P * j, loads - 1u);
+                    const unsigned e = q * 64u + lane;
+                    const std::uint32_t b = min(b0 + e / kMp, a.blocks - 1u);
+                    lds_load4(from + static_cast<std::uint64_t>(b) * kMp + e % kMp, base + at + q * 256u);
+                }
+            };
+            per_block(a.block_sums, kSumLoads, kXBytes);
+            per_block(a.inv_scale, kInvLoads, kInvAt);
         };
 #pragma unroll
         for (unsigned c = 0; c + 1u < kBuffers; ++c) fill(c);
@@ -383,6 +401,7 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
     // or four activation tiles, whose registers hold no more.
     half8v frag[2][MT][kParts];
     float4v sums[kSums ? MT : 1];
+    float4v invs[BLOCKS ? MT : 1];
     const auto read_stage = [&]<unsigned q>(const unsigned char* base) __attribute__((always_inline)) {
         constexpr unsigned blk = q * kParts / 2u;
 #pragma unroll
@@ -415,12 +434,11 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
         float4v p2[FMT == kQ6_K ? TN : 1][FMT == kQ6_K ? MT : 1];
         if constexpr (!LAST || kParts == 1u) read_stage.template operator()<q + 1u>(base);
         const auto read_sums = [&]() __attribute__((always_inline)) {
-            if constexpr (kSums) {
 #pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    sums[t] = *reinterpret_cast<const float4v*>(
-                        base + kXBytes + (blk * kMp + static_cast<unsigned>(t) * 16u + 4u * (lane >> 4)) * 4u);
-                }
+            for (int t = 0; t < MT; ++t) {
+                const unsigned at = (blk * kMp + static_cast<unsigned>(t) * 16u + 4u * (lane >> 4)) * 4u;
+                if constexpr (kSums) sums[t] = *reinterpret_cast<const float4v*>(base + kXBytes + at);
+                if constexpr (BLOCKS) invs[t] = *reinterpret_cast<const float4v*>(base + kInvAt + at);
             }
         };
         if constexpr (kParts == 2u) read_sums();
@@ -489,16 +507,28 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
                 float4v& sum = L > 2u ? pair[j][t] : L > 1u ? part[j][t] : acc[j][t];
+                constexpr bool kFirst = L > 2u && blk % 4u == 0u;
+                const auto add = [&](const float4v& by, const float4v& v) __attribute__((always_inline)) {
+                    if constexpr (kFirst) sum = by * v;
+                    else sum += by * v;
+                };
+                const float4v w4{ws[j], ws[j], ws[j], ws[j]};
                 if constexpr (FMT == kF16) {
-                    if constexpr (L > 2u && blk % 4u == 0u) sum = p[j][t];
-                    else sum += p[j][t];
-                } else if constexpr (L > 2u && blk % 4u == 0u) {
-                    sum = ws[j] * p[j][t];
+                    add(invs[t], p[j][t]);
+                } else if constexpr (!BLOCKS) {
+                    add(w4, p[j][t]);
+                    if constexpr (kSums) sum -= wo[j] * sums[t];
+                } else if constexpr (FMT == kQ6_K) {
+                    float4v v = ws[j] * p[j][t];
+                    v += ws2[j] * p2[j][t];
+                    add(invs[t], v);
+                } else if constexpr (kSums) {
+                    add(invs[t], ws[j] * p[j][t] - wo[j] * sums[t]);
                 } else {
-                    sum += ws[j] * p[j][t];
+                    // A power of two scales without rounding, so this product
+                    // rounds once, as under a row's scale.
+                    add(w4, invs[t] * p[j][t]);
                 }
-                if constexpr (FMT == kQ6_K) sum += ws2[j] * p2[j][t];
-                if constexpr (kSums) sum -= wo[j] * sums[t];
                 if constexpr (L > 2u && blk % 4u == 3u) part[j][t] += sum;
             }
     };
@@ -596,9 +626,10 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
 
     // D[row = activation row][col = weight row], as skinny_kernel.
     if constexpr (SERIAL) flush_split();
-    else load_inv();
+    else if constexpr (!BLOCKS) load_inv();
     const auto value = [&](int j, int t, int i, float bn) __attribute__((always_inline)) {
         if constexpr (SERIAL) return total[j][t][i] + bn;
+        else if constexpr (BLOCKS) return acc[j][t][i] + bn;
         else return acc[j][t][i] * inv[t][i] + bn;
     };
     if constexpr (SWIGLU) {
@@ -663,32 +694,96 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
     }
 }
 
-template <int FMT, int MT, int TN, int W>
-hipError_t launch_w(const StreamArgs& a, std::uint32_t blocks, hipStream_t stream) {
+// The scales a format and width run with: rows of the tile formats at any
+// width; blocks always over dense rows, else at one activation tile and, Q8_0
+// on eight waves, two (stream_route's rule asks for no others).
+template <int FMT, int MT, int TN, int W, bool BLOCKS>
+constexpr bool kCompiled = dense_storage(FMT) ? BLOCKS
+                           : !BLOCKS || MT == 1 || (FMT == kQ8_0 && MT == 2 && TN == 1 && W == 8);
+
+template <int FMT, int MT, int TN, int W, bool BLOCKS>
+hipError_t launch_scaled(const StreamArgs& a, std::uint32_t blocks, hipStream_t stream) {
     const dim3 threads(64 * (W + kProducers));
-    if (a.ffn_tiles == 0u) {
-        hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, false, false>), dim3(blocks), threads, 0, stream, a);
+    if constexpr (!kCompiled<FMT, MT, TN, W, BLOCKS>) {
+        return hipErrorInvalidConfiguration;
+    } else if (a.ffn_tiles == 0u) {
+        hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, false, false, BLOCKS>), dim3(blocks), threads, 0, stream, a);
     } else if constexpr (dense_storage(FMT)) {
         return hipErrorInvalidConfiguration;
     } else if (a.serial > 1u) {
         if constexpr (FMT == kQ8_0 && MT == 2 && W == 10) {
-            hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, true, true>), dim3(blocks), threads, 0, stream, a);
+            hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, true, true, false>), dim3(blocks), threads, 0, stream, a);
         } else {
             return hipErrorInvalidConfiguration;
         }
     } else {
-        hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, true, false>), dim3(blocks), threads, 0, stream, a);
+        hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, true, false, BLOCKS>), dim3(blocks), threads, 0, stream, a);
     }
     return hipGetLastError();
+}
+
+template <int FMT, int MT, int TN, int W>
+hipError_t launch_w(const StreamArgs& a, const SkinnyShape& s, std::uint32_t blocks, hipStream_t stream) {
+    return s.block_scaled ? launch_scaled<FMT, MT, TN, W, true>(a, blocks, stream)
+                          : launch_scaled<FMT, MT, TN, W, false>(a, blocks, stream);
+}
+
+// One wave per 32-element block and 16-row tile: lane l holds row l % 16,
+// elements 8 (l / 16)..+7, the fragment's own order, so loads are whole 128-byte
+// runs and stores 1 KiB.  Rows past m and blocks past k are zeros.
+__global__ __launch_bounds__(256) void split_blocks_kernel(const float* __restrict__ x, std::uint32_t m, std::uint64_t k,
+                                                           std::uint32_t blocks, std::uint32_t mtiles,
+                                                           u32x4* __restrict__ xs, float* __restrict__ block_sums,
+                                                           float* __restrict__ inv_scale) {
+#pragma clang fp contract(off)
+    const std::uint32_t lane = threadIdx.x & 63u;
+    const std::uint32_t w = blockIdx.x * 4u + (threadIdx.x >> 6);
+    if (w >= blocks * mtiles) return;
+    const std::uint32_t b = w / mtiles, t = w % mtiles;
+    const std::uint32_t row = t * 16u + (lane & 15u);
+    float v[8];
+    const std::uint64_t col = static_cast<std::uint64_t>(b) * 32u + 8u * (lane >> 4);
+    if (row < m && col < k) {
+        const float4v* src = reinterpret_cast<const float4v*>(x + static_cast<std::uint64_t>(row) * k + col);
+        const float4v lo = src[0], hi = src[1];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = lo[e];
+            v[4 + e] = hi[e];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+    }
+    float amax = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[e]));
+    amax = fmaxf(amax, __shfl_xor(amax, 16));
+    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    float s, inv;
+    block_scale(amax, s, inv);
+    half8v hi, lo;
+    split8(v, s, hi, lo);
+    const float sum01 = v[0] * s + v[1] * s, sum23 = v[2] * s + v[3] * s;
+    const float sum45 = v[4] * s + v[5] * s, sum67 = v[6] * s + v[7] * s;
+    float sum = (sum01 + sum23) + (sum45 + sum67);
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    xs[static_cast<std::uint64_t>(w) * 128u + lane] = __builtin_bit_cast(u32x4, hi);
+    xs[static_cast<std::uint64_t>(w) * 128u + 64u + lane] = __builtin_bit_cast(u32x4, lo);
+    if (lane < 16u) {
+        block_sums[static_cast<std::uint64_t>(b) * mtiles * 16u + row] = sum;
+        inv_scale[static_cast<std::uint64_t>(b) * mtiles * 16u + row] = inv;
+    }
 }
 
 template <int FMT, int MT>
 hipError_t launch_mt(const StreamArgs& a, const SkinnyShape& s, std::uint32_t blocks, hipStream_t stream) {
     if constexpr (!(FMT == kQ6_K && MT >= 3)) {
-        if (s.waves == 10u && s.tile_n == 2u) return launch_w<FMT, MT, 2, 10>(a, blocks, stream);
+        if (s.waves == 10u && s.tile_n == 2u) return launch_w<FMT, MT, 2, 10>(a, s, blocks, stream);
     }
-    if (s.waves == 10u && s.tile_n == 1u) return launch_w<FMT, MT, 1, 10>(a, blocks, stream);
-    if (s.waves == 8u && s.tile_n == 1u) return launch_w<FMT, MT, 1, 8>(a, blocks, stream);
+    if (s.waves == 10u && s.tile_n == 1u) return launch_w<FMT, MT, 1, 10>(a, s, blocks, stream);
+    if (s.waves == 8u && s.tile_n == 1u) return launch_w<FMT, MT, 1, 8>(a, s, blocks, stream);
     return hipErrorInvalidConfiguration;
 }
 
@@ -703,6 +798,16 @@ hipError_t launch_fmt(const StreamArgs& a, const SkinnyShape& s, std::uint32_t b
 }
 
 } // namespace
+
+hipError_t launch_split_activations_blocks(const float* x, std::uint32_t m, std::uint64_t k, std::uint64_t kp,
+                                           const SplitWorkspace& ws, hipStream_t stream) {
+    const std::uint64_t mtiles = ceil_div(m, 16u), waves = kp / 32u * mtiles;
+    if (m == 0u || m > 64u || k % 32u != 0u || waves > 0x7fffffffu) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(split_blocks_kernel, dim3(static_cast<unsigned>(ceil_div(waves, 4u))), dim3(256), 0, stream, x, m,
+                       k, static_cast<std::uint32_t>(kp / 32u), static_cast<std::uint32_t>(mtiles),
+                       static_cast<u32x4*>(ws.xs), ws.block_sums, ws.inv_scale);
+    return hipGetLastError();
+}
 
 bool stream_preferred(const TilePlanes& p, std::uint32_t m) {
     // Measured against the kernels it replaces on the Qwen2-7B matrices in the

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 import oracle
-from air_amd import capi
+from air_amd import capi, quant
 from tests import helpers
 from tests.test_gpu_dense import _weights
 
@@ -106,6 +106,70 @@ def test_stream_outliers_keep_small_channels(torch_cuda, hip_ctx):
         share = oracle.linear_row_list(capi.TYPE_Q4_0, canon, k, n, small, rows).astype(np.float64)
         for r in range(m):
             assert np.linalg.norm(got[r] - want[r]) <= 1e-3 * np.linalg.norm(share[r]), r
+    finally:
+        mat.release()
+
+
+# (format, K, N, M): the matrices the streaming kernel takes from kernels that
+# scale the activations per step or block -- from the wave-split kernel over f32
+# rows, the fused one (256 MiB of codes, up to four rows) and the dense one.
+BLOCK_CASES = [
+    (capi.TYPE_Q8_0, 2048, 16500, 8),
+    (capi.TYPE_Q8_0, 2048, 41000, 7),
+    (capi.TYPE_Q8_0, 4640, 1613, 28),
+    (capi.TYPE_Q8_0, 4096, 65600, 3),
+    (capi.TYPE_Q4_0, 2112, 34000, 5),
+    (capi.TYPE_Q4_0, 2048, 17000, 16),
+    (capi.TYPE_Q4_K, 2304, 17000, 12),
+    (capi.TYPE_Q4_K, 8448, 1530, 8),
+    (capi.TYPE_Q6_K, 8448, 1530, 13),
+    (capi.TYPE_Q6_K, 2048, 41000, 20),
+    (capi.TYPE_Q6_K, 2304, 4200, 40),
+    (capi.TYPE_Q6_K, 2304, 4200, 64),
+    (capi.TYPE_F16, 2048, 41000, 24),
+    (capi.TYPE_F16, 3104, 4200, 33),
+    (capi.TYPE_F16, 8224, 1530, 64),
+]
+
+
+@pytest.mark.parametrize("type_id,k,n,m", BLOCK_CASES, ids=[f"{capi.TYPE_NAMES[c[0]]}-{c[2]}x{c[1]}-{c[3]}" for c in BLOCK_CASES])
+def test_stream_keeps_blocks_beside_a_large_one(torch_cuda, hip_ctx, type_id, k, n, m):
+    """A channel 1e7 times the rest whose weights are zero: the outputs are the
+    other channels', and each row is within 6e-7 of the oracle -- the split's
+    truncation (below 2^-21 of a value, 1.2e-7 in the mean square) and f32 sums
+    (about 1.6e-7) with a factor of two; twice that in Q4_K, whose products are
+    of codes 0..15, about twice the weights, before their offset comes off.
+    Under one scale per row their low parts would be subnormal and the error
+    2e-5."""
+    torch = torch_cuda
+    dense = type_id in (capi.TYPE_Q6_K, capi.TYPE_F16)
+    if dense:
+        canon = _weights(type_id, k, n, seed=k + n)
+    else:
+        canon = quant.synthetic_weights_device(type_id, k, n, k + n, torch.device("cuda:0"), 0.02).cpu().numpy().reshape(-1)
+    rows_view = canon.reshape(n, -1)
+    if type_id == capi.TYPE_F16:
+        rows_view[:, :64] = 0
+    elif type_id == capi.TYPE_Q6_K:
+        rows_view[:, 208:210] = 0
+    else:
+        rows_view[:, :4 if type_id == capi.TYPE_Q4_K else 2] = 0
+    mat = capi.Matrix(hip_ctx, type_id, k, n, canon, canon.nbytes, on_device=False)
+    rows = np.unique(np.concatenate([np.arange(0, n, max(1, n // 200)), np.arange(n - 20, n)])).astype(np.uint64)
+    try:
+        plan = mat.plan(m)
+        print(f"blocks {capi.TYPE_NAMES[type_id]} {n}x{k} M={m}: {plan}", flush=True)
+        assert "stream_kernel" in plan, plan
+        x = helpers.activations(m, k, seed=m + k)
+        x[:, 5] = 1e7 * np.where(np.arange(m) % 2 == 0, 1.0, -1.0)
+        y = torch.empty((m, n), dtype=torch.float32, device="cuda:0")
+        mat.linear(torch.from_numpy(x).to("cuda:0"), y, m)
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()[:, rows.astype(np.int64)]
+        want = oracle.linear_row_list(type_id, canon, k, n, x, rows)
+        errors = [helpers.rel_l2(got[r], want[r]) for r in range(m)]
+        print(f"blocks error {max(errors):.2e}", flush=True)
+        assert max(errors) <= (1.2e-6 if type_id == capi.TYPE_Q4_K else 6e-7), plan
     finally:
         mat.release()
 
