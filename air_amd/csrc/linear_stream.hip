@@ -191,13 +191,13 @@ __device__ __forceinline__ void load_dense_record(const StreamArgs& a, std::uint
         out.s = *reinterpret_cast<const u32x4*>(rec + 192u);
         out.d = static_cast<const std::uint16_t*>(a.scales)[blk];
     } else {
-        // A row that ends on the first block of a step has no second one.
+        // A row that ends on the first block of a step has no second one: the
+        // first again, not used (half_step).  Nothing here may touch what is
+        // loaded, or the wave waits for this record instead of its oldest.
         const std::uint64_t col = static_cast<std::uint64_t>(unit) * kStepK + 8u * g;
         const unsigned char* at = base + (row * a.k + col) * 2u;
-        const bool both = col + 32u < a.k;
         out.v[0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(at));
-        out.v[1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(at + (both ? 64u : 0u)));
-        if (!both) out.v[1] = u32x4{0u, 0u, 0u, 0u};
+        out.v[1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(at + (col + 32u < a.k ? 64u : 0u)));
     }
 }
 
@@ -424,8 +424,10 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
     // The products of block `blk` of a chunk, block b of step `sub` of a
     // record: every tile's high parts, then the low parts on top, so that
     // neighbouring MFMAs do not depend on each other.  LAST: the chunk's last.
+    // absent: the block lies past the row.
     const auto compute = [&]<unsigned blk, unsigned sub, unsigned b, bool LAST>(
-                             const unsigned char* base, const Record<FMT>(&w_in)[TN]) __attribute__((always_inline)) {
+                             const unsigned char* base, const Record<FMT>(&w_in)[TN], bool absent)
+                             __attribute__((always_inline)) {
         constexpr unsigned q = blk * 2u / kParts;       // the block's first stage
         half8v w[TN];
         float ws[TN], wo[TN];
@@ -446,7 +448,8 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             if constexpr (FMT == kF16) {
-                w[j] = __builtin_bit_cast(half8v, w_in[j].v[b]);
+                const u32x4 none{0u, 0u, 0u, 0u};
+                w[j] = __builtin_bit_cast(half8v, absent ? none : w_in[j].v[b]);
             } else if constexpr (FMT == kQ6_K) {
                 // Half `sub / 2`, quadrant 2 (sub % 2) + b: dwords {low
                 // nibbles of even, odd quadrants, high pairs} per
@@ -563,7 +566,9 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
 #pragma unroll
             for (int t = 0; t < MT; ++t) total[j][t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    // One trip: kBody steps from s.  WHOLE: all of them lie in the range.
+    // F16 rows of an odd number of blocks: the last step is half a one.
+    const bool half_step = FMT == kF16 && s_end == a.steps && a.k % kStepK != 0u;
+    // One trip: kBody steps from s.  WHOLE: all of them, in full, lie in the range.
     std::uint32_t buffer = 0u;
     bool first_half = true;   // kHold: of the second level's eight steps
     const auto trip = [&](std::uint32_t s, auto whole_tag) __attribute__((always_inline)) {
@@ -594,8 +599,9 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
                 if constexpr (SERIAL) {
                     if (s + i == flush) flush_split();
                 }
-                compute.template operator()<2u * cs, i % U, 0, false>(cur, ring[(i / U) % D]);
-                compute.template operator()<2u * cs + 1u, i % U, 1, cs + 1u == C>(cur, ring[(i / U) % D]);
+                compute.template operator()<2u * cs, i % U, 0, false>(cur, ring[(i / U) % D], false);
+                compute.template operator()<2u * cs + 1u, i % U, 1, cs + 1u == C>(
+                    cur, ring[(i / U) % D], FMT == kF16 && !WHOLE && half_step && s + i + 1u == s_end);
             }
             if constexpr (i % U == U - 1u) load_w(ring[(i / U) % D], (s + i) / U + D);
             __builtin_amdgcn_sched_barrier(0);
@@ -614,7 +620,7 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
         if constexpr (kHold) first_half = !first_half;
     };
     std::uint32_t s = s_begin;
-    for (; s + kBody <= s_end; s += kBody) trip(s, std::true_type{});
+    for (; s + kBody <= s_end - (half_step ? 1u : 0u); s += kBody) trip(s, std::true_type{});
     if (s < s_end) {
         trip(s, std::false_type{});
     } else if (kHold && !first_half) {

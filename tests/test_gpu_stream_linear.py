@@ -83,6 +83,37 @@ def test_stream_linear(torch_cuda, hip_ctx, type_id, k, n, ms):
         mat.release()
 
 
+@pytest.mark.parametrize("k,m", [(3104, 20), (4064, 20), (4064, 40), (4064, 64), (3616, 33)])
+def test_stream_f16_half_step(torch_cuda, hip_ctx, k, m):
+    """F16 rows of an odd number of 32-blocks, their last step at the start, the
+    end and the middle of a trip: an infinite weight in the last block reaches
+    its own output as an infinity (not a NaN: the block past the row is left
+    out, not multiplied by zeros) and no other."""
+    torch = torch_cuda
+    n = 4200
+    canon = _weights(capi.TYPE_F16, k, n, seed=k)
+    w = canon.view(np.float16).reshape(n, k)
+    w[70, k - 1] = np.inf
+    w[n - 1, k - 9] = -np.inf
+    mat = capi.Matrix(hip_ctx, capi.TYPE_F16, k, n, canon, canon.nbytes, on_device=False)
+    try:
+        assert "stream_kernel" in mat.plan(m), mat.plan(m)
+        x = helpers.activations(m, k, seed=m)
+        x[:, k - 9] = x[:, k - 1] = 1.2345678      # hi and lo parts both non-zero
+        rows = np.unique(np.concatenate([np.arange(0, n, 40), [70, n - 1]])).astype(np.uint64)
+        y = torch.empty((m, n), dtype=torch.float32, device="cuda:0")
+        mat.linear(torch.from_numpy(x).to("cuda:0"), y, m)
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()
+        assert (got[:, 70] == np.inf).all() and (got[:, n - 1] == -np.inf).all(), mat.plan(m)
+        finite = rows[(rows != 70) & (rows != n - 1)]
+        want = oracle.linear_row_list(capi.TYPE_F16, canon, k, n, x, finite)
+        for r in range(m):
+            assert helpers.rel_l2(got[r, finite.astype(np.int64)], want[r]) <= DENSE_TOL, (r, mat.plan(m))
+    finally:
+        mat.release()
+
+
 def test_stream_outliers_keep_small_channels(torch_cuda, hip_ctx):
     """A few channels 1e4 times the rest: the error against the small channels'
     own share of the output stays at 1e-3 (f32 rounding of the outputs)."""
