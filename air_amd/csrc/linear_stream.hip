@@ -815,47 +815,93 @@ hipError_t launch_split_activations_blocks(const float* x, std::uint32_t m, std:
     return hipGetLastError();
 }
 
+namespace {
+
+// Row tiles a workgroup takes (plan_stream's comment says why).
+std::uint32_t stream_tile_n(const TilePlanes& p, std::uint32_t m) {
+    return p.nt > 2560u && !(p.type == kQ6_K && m > 32u) ? 2u : 1u;   // (that one would spill)
+}
+std::uint32_t stream_waves(const TilePlanes& p) { return p.nt > 2048u ? 10u : 8u; }
+
+// Whether a wide matrix's workgroups fill their rounds of the CUs.  Twenty
+// tiles a workgroup (from 2561 row tiles) leave half of the CUs idle at first:
+// one round needs 160 workgroups (Q8_0, K = 3584 at 8 rows, time of the kernels
+// before over this: 3000 row tiles 0.85, 3200 1.02; at 33..48 rows 176, 3200
+// 0.95..0.98), several need the last to bring their slots to 78 % (5130 row
+// tiles, 50 %: 0.69..1.0; 7600, 74 %: 0.90..1.12; 8200, 80 %: 1.07..1.15;
+// 11500, 75 %: 0.86..1.15; 12800, 83 %: 1.0..1.16), Q8_0 at up to four rows to 88
+// % (8200 and 12800 0.95..0.97, 9504 1.04).
+bool stream_fills(const TilePlanes& p, std::uint32_t m) {
+    const std::uint64_t groups = ceil_div(p.nt, stream_waves(p) * stream_tile_n(p, m));
+    const bool q8 = p.type == kQ8_0;
+    if (groups <= 256u) return p.nt <= 2560u || groups >= (q8 && m > 32u && m <= 48u ? 176u : 160u);
+    return groups * 100u >= ceil_div(groups, 256u) * 256u * (q8 && m <= 4u ? 88u : 78u);
+}
+
+} // namespace
+
 bool stream_preferred(const TilePlanes& p, std::uint32_t m) {
-    // Measured against the kernels it replaces on the Qwen2-7B matrices in the
-    // tile formats at M = 3, 8, 16, 20, 32, 48 and 64 (graph replay, split
-    // launch included; the table at the top):
-    //  * wide matrices (over 1024 row tiles): faster at every width, but for
-    //    Q8_0 ones of 2000..4096 row tiles at 17..32 rows, whose eight-wave
-    //    plan and its two splits stay;
-    //  * narrow ones at two or more activation tiles: faster on q|k|v (1-2 us)
-    //    and, K being long, on down (2-9 us; Q8_0 from 25 rows: 33.3 against
-    //    32.6 us at 20); the matrices the wave-split kernel takes with short K
-    //    (o) keep it (16.5 against 14.5 us at 32 rows);
-    //  * narrow ones at one activation tile: only Q4_K with long K (down 31.1
-    //    -> 25.5 us at 8 rows; Q8_0 28.0 against 24.8, Q4_0 even).
+    // Measured against the kernels it replaces (graph replay over 400 MB of
+    // copies, split launch included) in every format at 3, 8, 16, 20, 26, 32,
+    // 40, 56 and 64 rows: 30 counts of row tiles from 1032 to 12800 at K = 2048
+    // and 3584, 15 from 96 to 1000 at K = 2048, 3584, 4352, 8192 and 18944.
+    // Taken where it is faster or even; figures are old time over new.
+    //  * wide matrices (over 1024 row tiles) whose workgroups fill their
+    //    rounds (stream_fills): 1.0..1.4, but for Q8_0 ones of 2000..4096 row
+    //    tiles at 17..32 rows, whose eight-wave plan and its two splits stay,
+    //    and short K at up to four rows (0.96 at 1900 row tiles of 2048) or, in
+    //    several rounds, from 49 (0.92..0.98);
+    //  * 257..1024 row tiles at two or more activation tiles: 1.0..1.4 from K =
+    //    3584 on.  At K = 2048 the K splits that fill the GPU cost more than
+    //    they stream: Q8_0 0.77..1.0, Q4_0 0.75..0.95 up to 640 row tiles;
+    //  * up to 256 row tiles with long K at two or more (the wave-split kernel
+    //    keeps short K): 1.0..1.4; Q8_0 at two only from 25 rows, 128 row tiles
+    //    and K = 8192 (K = 4352 0.94..0.98, 96 row tiles of 18944 0.94);
+    //  * at four activation tiles the K splits of the skinny kernel can fill
+    //    its two workgroups a CU; then it is as fast up to K = 8192 (Q8_0 512
+    //    row tiles of 3584 0.92, 256 of 8192 0.96, Q4_0 0.95..1.0);
+    //  * at one activation tile only Q4_K with long K (1.1..2.2);
+    //  * fewer than 128 row tiles only with K over 8192 (96 of 8192: Q8_0 0.84,
+    //    Q4_0 0.95, Q4_K 0.92 at 8 rows, 1.2 at 3).
     // Short K (under 32 steps) leaves the ring and the chunks nothing to run
-    // ahead of, and under 96 row tiles the K splits that would fill the GPU
-    // cost more than they stream (33 tiles of K = 8448 at 6 rows: 23.6 us on
-    // the wave-split kernel, 31.6 here).
-    if (m < 2u || m > 64u || p.kp / kStepK < 32u) return false;
+    // ahead of, and so do fewer than 96 row tiles.
+    if (m < 2u || m > 64u || p.kp / kStepK < 32u || p.nt < 96u) return false;
     const bool one = m <= 16u, two = !one && m <= 32u;
+    const bool wide = p.nt > 1024u, long_k = p.k > 4096u;
     if (p.type == kQ6_K) {
-        // Against dense_mfma_kernel: 1.1 to 3.5 times faster but for narrow
-        // short-K matrices below 16 rows (o at 13 rows 14.7 against 15.2 us).
-        return p.nt >= 96u && (m >= 16u || p.nt > 256u || p.k > 4096u);
+        // Against dense_mfma_kernel: 1.1 to 5.6 times faster but for narrow
+        // short-K matrices below 16 rows (o at 13 rows 14.7 against 15.2 us),
+        // or below 33 of K = 2048 (0.81..0.97).
+        return p.nt > 256u || long_k || m > 32u || (m >= 16u && p.k >= 3072u);
     }
     if (p.type == kF16) {
         // Against dense_mfma_kernel, which reads the weights once for 64 rows
-        // too but from half the waves: from 17 rows (gate|up at 24 99 -> 79
-        // us, 13 even; down 79 -> 59), later on narrow (o at 48 rows 28.5
-        // against 29.2) and short-K ones (688 tiles of K = 2048 at 24 rows
-        // 28.6 against 30.0, at 48 46 -> 33).
-        if (m <= 16u || p.nt < 96u) return false;
-        if (two) return p.nt > 1024u || (p.nt > 256u && p.k >= 3072u) || p.k > 8192u;
-        return p.nt > 256u || p.k > 4096u || m > 48u;
+        // too but from half the waves: from 33 rows 1.5..4.8 times faster but
+        // for narrow short-K matrices below 49; at 17..32 1.0..2.9 where the
+        // rounds are filled (3000 row tiles 0.9) and K is not short (1400 row
+        // tiles of 2048 0.94).
+        if (one) return false;
+        if (two) return stream_fills(p, m) && (p.nt > 1700u || (p.nt > 256u && p.k >= 3072u) || p.k > 8192u);
+        return p.nt > 256u || long_k || m > 48u;
     }
-    if (p.nt > 1024u) return !(p.type == kQ8_0 && two && p.nt >= 2000u && p.nt <= 4096u);
-    if (p.nt < 96u) return false;
-    const bool long_k = p.k > 4096u;
+    if (wide) {
+        if (p.type == kQ8_0 && two && p.nt >= 2000u && p.nt <= 4096u) return false;
+        if (p.type == kQ8_0 && p.k < 3072u && ((m <= 4u && p.nt <= 2048u) || (m > 48u && p.nt > 5120u))) return false;
+        return stream_fills(p, m);
+    }
+    if (p.nt < 128u && p.k <= 8192u && !(one && m <= 4u)) return false;
     if (one) return p.type == kQ4_K && long_k;
-    if (p.nt > 256u) return true;
+    if (m > 48u && p.type != kQ4_K && p.k <= 8192u) {
+        const SkinnyShape s = plan_skinny(p, m, 0u, 0u);
+        if (s.groups * s.splits >= 384u) return false;
+    }
+    if (p.nt > 256u) {
+        const std::uint32_t least = p.type == kQ8_0 ? 1025u : p.type == kQ4_0 ? 800u : 0u;   // row tiles at short K
+        return p.k >= 3072u || p.nt >= least;
+    }
     if (p.type == kQ4_K && !two && p.k < 8192u) return false;   // even or slower at 33..64 rows (27.7, 28.2 us)
-    return long_k && (p.type != kQ8_0 || m > 24u);
+    if (p.type == kQ8_0 && two) return m > 24u && p.k >= 8192u && p.nt >= 128u;
+    return long_k;
 }
 
 SkinnyShape plan_stream(const TilePlanes& p, std::uint32_t m) {
@@ -867,8 +913,8 @@ SkinnyShape plan_stream(const TilePlanes& p, std::uint32_t m) {
     // workgroup, ten from 2049 row tiles, twenty (two per wave, which also
     // halves the activations read per tile: lm_head 141 -> 121 us at 32 rows)
     // from 2561, where ten would start a second round.
-    s.tile_n = p.nt > 2560u && !(p.type == kQ6_K && s.mt >= 3u) ? 2u : 1u;   // (that one would spill)
-    s.waves = p.nt > 2048u ? 10u : 8u;
+    s.tile_n = stream_tile_n(p, m);
+    s.waves = stream_waves(p);
     s.groups = static_cast<std::uint32_t>(ceil_div(p.nt, s.waves * s.tile_n));
     // Otherwise K is split over workgroups up to that round, at least twelve
     // steps each (the partials' round trip: Q8_0 q|k|v at 32 rows 16.9 us with
@@ -954,8 +1000,13 @@ bool plan_stream_swiglu(const TilePlanes& p, std::uint32_t m, const SkinnyShape&
     } else {
         // Q8_0 at 17..32 rows, 2000..4096 row tiles: the plain linear keeps
         // the eight-wave kernel (37.8 us; its two splits reduce in another
-        // 5 with the SwiGLU); here its splits are summed in the workgroup.
-        if (p.type != kQ8_0 || m <= 16u || m > 32u || p.nt < 2000u || p.nt > 4096u || p.kp / kStepK < 32u) return false;
+        // 5 with the SwiGLU); here its splits are summed in the workgroup,
+        // where the workgroups fill the GPU (2800 row tiles 0.84..0.99 times
+        // the reduction's speed).
+        if (p.type != kQ8_0 || m <= 16u || m > 32u || p.nt < 2000u || p.nt > 4096u || p.kp / kStepK < 32u ||
+            !stream_fills(p, m)) {
+            return false;
+        }
         s = linear;
         s.stream = true;
         s.waves = 10u;
