@@ -926,6 +926,7 @@ PrefillShape plan_prefill(const TilePlanes& p, std::uint32_t m, const PrefillTun
         // tiles, 43.5 us split 2 ways, 50.5 unsplit).
         const std::uint64_t tiles = static_cast<std::uint64_t>(s.m_tiles) * s.groups;
         const std::uint64_t cus = tuning.cus ? tuning.cus : 256u, slots = 2u * cus;
+        const bool four_bit = p.type == kQ4_0 || p.type == kQ4_K;
         splits = 1u;
         while (tiles * splits * 2u <= 640u && s.steps / (splits * 2u) >= 16u) splits *= 2u;
         if (s.tile_m == 4u && s.tile_n == 2u) {
@@ -934,7 +935,13 @@ PrefillShape plan_prefill(const TilePlanes& p, std::uint32_t m, const PrefillTun
             // and 301: Q8_0 27.5 -> 21.7, 29.2 -> 25.6, 31.2 -> 27.7 and
             // 33.3 -> 29.8 us, Q4_K 39.9 -> 34.8 at 301; six splits are no
             // better than four at 96 (22.3).
-            splits = std::max<std::uint32_t>(splits, static_cast<std::uint32_t>(std::min<std::uint64_t>(slots / tiles, s.steps / 14u)));
+            // The 4-bit formats keep a power of two that gives nearly every CU
+            // its workgroup where more would give only some a second (K = 5120,
+            // 56 and 64 tiles at 5 splits against 4: Q4_K 0.93..0.96 times the
+            // speed, Q4_0 0.97..1.0; Q8_0 and F16 1.0..1.07).
+            const std::uint64_t more = std::min<std::uint64_t>(slots / tiles, s.steps / 14u);
+            const bool some = four_bit && tiles * splits * 8u >= cus * 7u && tiles * splits <= cus && tiles * more * 4u <= cus * 5u;
+            if (!some) splits = std::max<std::uint32_t>(splits, static_cast<std::uint32_t>(more));
         } else if (s.tile_m == 8u && s.tile_n == 4u && tiles <= slots) {
             // At most the two workgroups a CU holds, and of those counts the
             // one whose last workgroup per CU is missing least often: down
@@ -944,7 +951,11 @@ PrefillShape plan_prefill(const TilePlanes& p, std::uint32_t m, const PrefillTun
             // a workgroup stays unless the other count fills a quarter more of
             // the slots: at 512 rows 9 splits (504 workgroups) took 99.8 us, 8
             // (448) 101.1, for an eighth more partials.  More tiles than CUs
-            // stay whole: gate|up at 256 rows paid for 78 MB of partials.
+            // stay whole: gate|up at 256 rows paid for 78 MB of partials; but
+            // in the 4-bit formats not while two splits' partials (16 bytes a
+            // row and output) are small beside K (37888 x 8192: at 130 rows
+            // Q4_0 220 us split, 246 whole, at 200 even; Q8_0 1.03 the other
+            // way).
             const auto fill = [&](std::uint64_t n) { return tiles * n * 1024u / (ceil_div(tiles * n, cus) * cus); };
             const std::uint64_t power = splits;
             std::uint64_t best = 1u;
@@ -952,7 +963,9 @@ PrefillShape plan_prefill(const TilePlanes& p, std::uint32_t m, const PrefillTun
                 if (fill(n) >= fill(best)) best = n;
             }
             const bool covers = tiles * power <= slots && tiles * power >= cus;
-            splits = static_cast<std::uint32_t>(covers && fill(best) * 4u <= fill(power) * 5u ? power : best);
+            const bool keep = (covers && fill(best) * 4u <= fill(power) * 5u) ||
+                              (four_bit && tiles > cus && 48u * static_cast<std::uint64_t>(m) <= p.k);
+            splits = static_cast<std::uint32_t>(keep ? power : best);
         }
     }
     // A grid of 8x4 tiles (two workgroups per CU) that ends in a round less

@@ -607,3 +607,24 @@ def test_prefill_fill_splits(torch_cuda, hip_ctx, type_id, k, n, m, splits):
         assert helpers.rel_l2(got[sample][:, rows.astype(np.int64)], want) < PREFILL_EXPECT, plan
     finally:
         mat.release()
+
+
+# (format, K, N, M, splits): plans alone.  4-bit formats beside Q8_0: a power of
+# two that gives nearly every CU a workgroup, and more tiles than CUs at long K.
+SPLIT_PLANS = [
+    (capi.TYPE_Q4_K, 5120, 2048, 200, 4), (capi.TYPE_Q4_0, 5120, 3584, 96, 4), (capi.TYPE_Q8_0, 5120, 2048, 200, 5),
+    (capi.TYPE_Q4_K, 5120, 4608, 66, 5), (capi.TYPE_Q4_0, 8192, 37888, 130, 2), (capi.TYPE_Q4_0, 8192, 37888, 200, 1),
+    (capi.TYPE_Q8_0, 8192, 37888, 130, 1),
+]
+
+
+@pytest.mark.parametrize("type_id,k,n,m,splits", SPLIT_PLANS)
+def test_prefill_split_plans(torch_cuda, hip_ctx, type_id, k, n, m, splits):
+    elements, size = helpers.BLOCK[type_id]
+    zeros = torch_cuda.zeros(n * (k // elements) * size, dtype=torch_cuda.uint8, device="cuda:0")
+    mat = capi.Matrix(hip_ctx, type_id, k, n, zeros, zeros.numel(), on_device=True)
+    try:
+        plan = mat.plan(m, tactic=capi.LINEAR_PREFILL)
+        assert re.search(r" splits=(\d+)", plan).group(1) == str(splits), plan
+    finally:
+        mat.release()
