@@ -785,7 +785,7 @@ __global__ __launch_bounds__(256) void split_blocks_kernel(const float* __restri
 
 template <int FMT, int MT>
 hipError_t launch_mt(const StreamArgs& a, const SkinnyShape& s, std::uint32_t blocks, hipStream_t stream) {
-    if constexpr (!(FMT == kQ6_K && MT >= 3)) {
+    if constexpr (!(FMT == kQ6_K && MT >= 3) && !(FMT == kF16 && MT >= 4)) {
         if (s.waves == 10u && s.tile_n == 2u) return launch_w<FMT, MT, 2, 10>(a, s, blocks, stream);
     }
     if (s.waves == 10u && s.tile_n == 1u) return launch_w<FMT, MT, 1, 10>(a, s, blocks, stream);
@@ -817,9 +817,12 @@ hipError_t launch_split_activations_blocks(const float* x, std::uint32_t m, std:
 
 namespace {
 
-// Row tiles a workgroup takes (plan_stream's comment says why).
+// Row tiles a workgroup takes (plan_stream's comment says why).  Not two per
+// wave where that would spill (Q6_K at three activation tiles) or leave no
+// registers for a second level of the K sum that the kernel replaced had (F16 at
+// four: 2.0e-7 from 64 bits at K = 2048, 1.6e-7 before and with one).
 std::uint32_t stream_tile_n(const TilePlanes& p, std::uint32_t m) {
-    return p.nt > 2560u && !(p.type == kQ6_K && m > 32u) ? 2u : 1u;   // (that one would spill)
+    return p.nt > 2560u && !(p.type == kQ6_K && m > 32u) && !(p.type == kF16 && m > 48u) ? 2u : 1u;
 }
 std::uint32_t stream_waves(const TilePlanes& p) { return p.nt > 2048u ? 10u : 8u; }
 

@@ -138,6 +138,40 @@ def test_stream_f16_half_step(torch_cuda, hip_ctx, k, m):
         mat.release()
 
 
+# (format, K, N, widths): long unsplit K, where a single running sum would show.
+SUM_CASES = [
+    (capi.TYPE_F16, 16384, 41000, (48, 64)),
+    (capi.TYPE_F16, 16384, 33000, (64,)),
+]
+
+
+@pytest.mark.parametrize("type_id,k,n,ms", SUM_CASES)
+def test_stream_k_sum_in_levels(torch_cuda, hip_ctx, type_id, k, n, ms):
+    """Relative L2 against float64 products at K = 16384 unsplit: 3e-7 = the
+    split's truncation (1.2e-7) and a K sum in levels of 8 and 64 blocks (about
+    1.5e-7), with a third to spare; one running sum of its 512 blocks is 4.3e-7."""
+    torch = torch_cuda
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(k + n)
+    w = torch.empty((n, k), dtype=torch.float16, device="cuda:0").normal_(0.0, 0.02, generator=gen)
+    mat = capi.Matrix(hip_ctx, type_id, k, n, w.view(torch.uint8), n * k * 2, on_device=True)
+    sample = torch.arange(0, n, n // 500, device="cuda:0")
+    ws = w[sample].double().T.contiguous()
+    try:
+        for m in ms:
+            plan = mat.plan(m)
+            assert "stream_kernel" in plan and " splits=1 " in plan + " ", plan
+            x = torch.randn((m, k), generator=gen, device="cuda:0")
+            y = torch.empty((m, n), dtype=torch.float32, device="cuda:0")
+            mat.linear(x, y, m)
+            want = x.double() @ ws
+            error = float((y[:, sample].double() - want).norm() / want.norm())
+            print(f"levels {capi.TYPE_NAMES[type_id]} {n}x{k} M={m} {error:.2e}: {plan}", flush=True)
+            assert error <= 3e-7, (m, error, plan)
+    finally:
+        mat.release()
+
+
 def test_stream_outliers_keep_small_channels(torch_cuda, hip_ctx):
     """A few channels 1e4 times the rest: the error against the small channels'
     own share of the output stays at 1e-3 (f32 rounding of the outputs)."""
