@@ -887,6 +887,12 @@ bool stream_preferred(const TilePlanes& p, std::uint32_t m) {
         if (two) return stream_fills(p, m) && (p.nt > 1700u || (p.nt > 256u && p.k >= 3072u) || p.k > 8192u);
         return p.nt > 256u || long_k || m > 48u;
     }
+    if (p.type == kQ4_K && m > 32u &&
+        plan_stream(p, m).steps_per_split * 16u > plan_skinny(p, m, 0u, 0u).steps_per_split * 17u) {
+        // A longer running sum than it replaces; a sixteenth longer measures
+        // even (K = 3584..18944: -6..+1.3 % of the error), a twelfth 2 % more.
+        return false;
+    }
     if (wide) {
         if (p.type == kQ8_0 && two && p.nt >= 2000u && p.nt <= 4096u) return false;
         if (p.type == kQ8_0 && p.k < 3072u && ((m <= 4u && p.nt <= 2048u) || (m > 48u && p.nt > 5120u))) return false;
@@ -930,6 +936,16 @@ SkinnyShape plan_stream(const TilePlanes& p, std::uint32_t m) {
     splits = std::max(splits, 1u);
     const std::uint32_t unit = p.type == kQ8_0 || p.type == kF16 ? 1u : p.type == kQ4_0 ? 2u : 4u;   // kUnit
     s.steps_per_split = static_cast<std::uint32_t>(ceil_div(ceil_div(s.steps, splits), unit) * unit);
+    // Q4_K at three and four activation tiles keeps one running sum a split
+    // (kLevels), so no split may be longer than the skinny kernel's: whole
+    // records go down, not up, where the extra split has its workgroups (down
+    // at 64 rows, 40 steps 4.04e-7 from 64 bits, 36 3.96e-7, the skinny
+    // kernel's 37 3.97e-7).
+    const std::uint32_t down = static_cast<std::uint32_t>(ceil_div(s.steps, splits) / unit * unit);
+    if (p.type == kQ4_K && s.mt >= 3u && splits > 1u && down > 0u && down < s.steps_per_split &&
+        s.groups * ceil_div(s.steps, down) <= 256u) {
+        s.steps_per_split = down;
+    }
     s.splits = static_cast<std::uint32_t>(ceil_div(s.steps, s.steps_per_split));
     return s;
 }

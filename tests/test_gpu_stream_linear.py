@@ -138,6 +138,22 @@ def test_stream_f16_half_step(torch_cuda, hip_ctx, k, m):
         mat.release()
 
 
+@pytest.mark.parametrize("k,n,m,splits", [(18944, 3584, 64, 9), (18944, 3584, 40, 9), (8448, 11008, 40, 2),
+                                          (2304, 6656, 64, 0), (4608, 4096, 40, 0), (3584, 37888, 48, 1)])
+def test_stream_q4_k_split_lengths(torch_cuda, hip_ctx, k, n, m, splits):
+    """Q4_K at 33..64 rows keeps one running sum a split: whole records round
+    down where the GPU has room for one more split, and where a split would be
+    over a sixteenth longer than the skinny kernel's that one stays (0)."""
+    zeros = torch_cuda.zeros(n * (k // 256) * 144, dtype=torch_cuda.uint8, device="cuda:0")
+    mat = capi.Matrix(hip_ctx, capi.TYPE_Q4_K, k, n, zeros, zeros.numel(), on_device=True)
+    try:
+        plan = mat.plan(m)
+        assert ("stream_kernel" in plan) == (splits != 0), plan
+        assert not splits or f" splits={splits}" in plan, plan
+    finally:
+        mat.release()
+
+
 # (format, K, N, widths): long unsplit K, where a single running sum would show.
 SUM_CASES = [
     (capi.TYPE_F16, 16384, 41000, (48, 64)),
