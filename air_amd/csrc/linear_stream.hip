@@ -293,10 +293,11 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
     constexpr unsigned D = kRing<FMT, MT, TN>;
     constexpr unsigned C = kChunk<MT>;
     constexpr unsigned L = SERIAL ? 1u : kLevels<FMT, MT, TN>;
-    // Steps per trip: the ring comes full circle.  At three levels the second
-    // one covers eight steps (two trips of four with four activation tiles,
-    // which would spill in a trip of eight).
-    constexpr bool kEight = L > 2u && MT <= 3;
+    // Steps per trip: the ring comes full circle.  At three levels, and at two
+    // where the ring is two steps (F16, three activation and two row tiles), the second one covers
+    // eight steps (two trips of four with four activation tiles, which would
+    // spill in a trip of eight).
+    constexpr bool kEight = (L > 2u && MT <= 3) || (L == 2u && FMT == kF16 && MT == 3 && TN == 2);
     constexpr unsigned kBody = D * U > C && D * U > (kEight ? 8u : 0u) ? D * U : kEight && C < 8u ? 8u : C;
     constexpr bool kHold = L > 2u && kBody < 8u;
     constexpr bool kSums = FMT == kQ4_K;

@@ -157,6 +157,7 @@ def test_stream_q4_k_split_lengths(torch_cuda, hip_ctx, k, n, m, splits):
 # (format, K, N, widths): long unsplit K, where a single running sum would show.
 SUM_CASES = [
     (capi.TYPE_F16, 16384, 41000, (48, 64)),
+    (capi.TYPE_F16, 16384, 51300, (24, 40)),
     (capi.TYPE_F16, 16384, 33000, (64,)),
 ]
 
@@ -164,8 +165,8 @@ SUM_CASES = [
 @pytest.mark.parametrize("type_id,k,n,ms", SUM_CASES)
 def test_stream_k_sum_in_levels(torch_cuda, hip_ctx, type_id, k, n, ms):
     """Relative L2 against float64 products at K = 16384 unsplit: 3e-7 = the
-    split's truncation (1.2e-7) and a K sum in levels of 8 and 64 blocks (about
-    1.5e-7), with a third to spare; one running sum of its 512 blocks is 4.3e-7."""
+    split's truncation (1.2e-7) and a K sum in levels (about 1.8e-7), with a third
+    to spare; one running sum of its 512 blocks is 4.3e-7."""
     torch = torch_cuda
     gen = torch.Generator(device="cuda:0")
     gen.manual_seed(k + n)
