@@ -261,11 +261,22 @@ constexpr unsigned kRing = FMT == kQ8_0 || FMT == kF16 ? (MT <= 2 ? 8u : 4u) / T
                            : FMT == kQ4_0 ? (MT <= 2 && TN == 1 ? 4u : 2u)
                                           : (TN == 1 && (FMT == kQ4_K || MT <= 2) ? 2u : 1u);   // Q4_K, Q6_K
 constexpr int kProducers = 2;
-// Levels of the K sum: three, or as many as leave no register in scratch.
+// Levels of the K sum: three at one and two activation tiles and for Q6_K, else
+// two (one where two would spill), one in the serial SwiGLU, whose plan has no
+// more.  Relative L2 from 64 bits at K = 3584 unsplit, the kernels replaced ->
+// this:
+//   three  Q8_0 at 8 rows 1.60e-7 -> 1.54e-7, Q4_0 1.58e-7 -> 1.54e-7, Q6_K at 64
+//          1.56e-7 -> 1.51e-7;
+//   two    Q8_0 lm_head at 40 rows 2.32e-7 -> 1.70e-7, F16 gate|up at 64 1.69e-7 ->
+//          1.66e-7;
+//   one    Q4_K from 33 rows (gate|up 4.40e-7 -> 4.27e-7, most of it from codes
+//          that start at 0), Q8_0 and Q4_0 at 49..64 with two row tiles a wave
+//          (lm_head 2.32e-7 either way: the kernel replaced has one too).
+// Q4_K at four activation and two row tiles and Q6_K at four activation tiles
+// keep one register in scratch.
 template <int FMT, int MT, int TN>
-constexpr unsigned kLevels = FMT == kF16 && MT == 2 && TN == 2              ? 2u
-                             : FMT == kQ6_K && (MT >= 3 || (MT == 2 && TN == 2)) ? 2u
-                             : MT <= 2                                         ? 3u
+constexpr unsigned kLevels = FMT == kF16 && MT == 2 && TN == 2      ? 2u
+                             : MT <= 2 || FMT == kQ6_K              ? 3u
                              : FMT == kQ4_K || (MT == 4 && TN == 2) ? 1u
                                                                     : 2u;
 
@@ -297,11 +308,12 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
     // where the ring is two steps (F16, three activation and two row tiles), the second one covers
     // eight steps (two trips of four with four activation tiles, which would
     // spill in a trip of eight).
-    constexpr bool kEight = (L > 2u && MT <= 3) || (L == 2u && FMT == kF16 && MT == 3 && TN == 2);
+    constexpr bool kEight = (L > 2u && MT <= (FMT == kQ6_K ? 2 : 3)) || (L == 2u && FMT == kF16 && MT == 3 && TN == 2);
     constexpr unsigned kBody = D * U > C && D * U > (kEight ? 8u : 0u) ? D * U : kEight && C < 8u ? 8u : C;
     constexpr bool kHold = L > 2u && kBody < 8u;
     constexpr bool kSums = FMT == kQ4_K;
     constexpr bool kDense = dense_storage(FMT);
+    constexpr bool kLateInv = FMT == kQ6_K && MT == 4;   // no registers to hold them through the MFMAs
     constexpr unsigned kMp = 16u * MT;
     constexpr unsigned kParts = MT <= 2 ? 2u : 1u;
     constexpr unsigned kFrags = 2u * C * 2u * MT;           // 1 KiB activation fragments per chunk
@@ -441,7 +453,7 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
             for (int t = 0; t < MT; ++t) {
                 const unsigned at = (blk * kMp + static_cast<unsigned>(t) * 16u + 4u * (lane >> 4)) * 4u;
                 if constexpr (kSums) sums[t] = *reinterpret_cast<const float4v*>(base + kXBytes + at);
-                if constexpr (BLOCKS) invs[t] = *reinterpret_cast<const float4v*>(base + kInvAt + at);
+                if constexpr (BLOCKS && !kLateInv) invs[t] = *reinterpret_cast<const float4v*>(base + kInvAt + at);
             }
         };
         if constexpr (kParts == 2u) read_sums();
@@ -512,6 +524,10 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
             for (int t = 0; t < MT; ++t) {
                 float4v& sum = L > 2u ? pair[j][t] : L > 1u ? part[j][t] : acc[j][t];
                 constexpr bool kFirst = L > 2u && blk % 4u == 0u;
+                if constexpr (kLateInv) {
+                    invs[t] = *reinterpret_cast<const float4v*>(
+                        base + kInvAt + (blk * kMp + static_cast<unsigned>(t) * 16u + 4u * (lane >> 4)) * 4u);
+                }
                 const auto add = [&](const float4v& by, const float4v& v) __attribute__((always_inline)) {
                     if constexpr (kFirst) sum = by * v;
                     else sum += by * v;
@@ -786,7 +802,7 @@ __global__ __launch_bounds__(256) void split_blocks_kernel(const float* __restri
 
 template <int FMT, int MT>
 hipError_t launch_mt(const StreamArgs& a, const SkinnyShape& s, std::uint32_t blocks, hipStream_t stream) {
-    if constexpr (!(FMT == kQ6_K && MT >= 3) && !(FMT == kF16 && MT >= 4)) {
+    if constexpr (!(FMT == kQ6_K && MT >= 2) && !(FMT == kF16 && MT >= 4)) {   // stream_tile_n
         if (s.waves == 10u && s.tile_n == 2u) return launch_w<FMT, MT, 2, 10>(a, s, blocks, stream);
     }
     if (s.waves == 10u && s.tile_n == 1u) return launch_w<FMT, MT, 1, 10>(a, s, blocks, stream);
@@ -818,12 +834,12 @@ hipError_t launch_split_activations_blocks(const float* x, std::uint32_t m, std:
 
 namespace {
 
-// Row tiles a workgroup takes (plan_stream's comment says why).  Not two per
-// wave where that would spill (Q6_K at three activation tiles) or leave no
-// registers for a second level of the K sum that the kernel replaced had (F16 at
-// four: 2.0e-7 from 64 bits at K = 2048, 1.6e-7 before and with one).
+// Row tiles a wave takes (plan_stream's comment says why).  Not two where the
+// registers then hold fewer levels of the K sum than the kernel replaced had
+// (from 64 bits at K = 2048, before / two tiles / one: F16 at four activation
+// tiles 1.6e-7 / 2.0e-7 / 1.6e-7, Q6_K at two 1.49e-7 / 1.52e-7 / 1.48e-7).
 std::uint32_t stream_tile_n(const TilePlanes& p, std::uint32_t m) {
-    return p.nt > 2560u && !(p.type == kQ6_K && m > 32u) && !(p.type == kF16 && m > 48u) ? 2u : 1u;
+    return p.nt > 2560u && !(p.type == kQ6_K && m > 16u) && !(p.type == kF16 && m > 48u) ? 2u : 1u;
 }
 std::uint32_t stream_waves(const TilePlanes& p) { return p.nt > 2048u ? 10u : 8u; }
 
