@@ -717,32 +717,37 @@ __global__ __launch_bounds__(64 * (W + kProducers), (W + kProducers + 3) / 4) vo
     }
 }
 
-// The scales a format and width run with: rows of the tile formats at any
-// width; blocks always over dense rows, else at one activation tile and, Q8_0
-// on eight waves, two (stream_route's rule asks for no others).
-template <int FMT, int MT, int TN, int W, bool BLOCKS>
-constexpr bool kCompiled = dense_storage(FMT) ? BLOCKS
-                           : !BLOCKS || MT == 1 || (FMT == kQ8_0 && MT == 2 && TN == 1 && W == 8);
+// What the rules reach.  Scales: blocks always over dense rows, else only at one
+// activation tile (Q4_K on eight waves) and, Q8_0 on eight waves, two; rows of
+// the tile formats at any width.  F16 from two activation tiles.  Ten waves of
+// one row tile over Q8_0 at two activation tiles only for the serial SwiGLU
+// (2049..2560 row tiles); no SwiGLU over matrices narrow enough for Q8_0's
+// blocks at two.
+template <int FMT, int MT, int TN, int W, bool SWIGLU, bool BLOCKS>
+constexpr bool kReached = dense_storage(FMT)           ? BLOCKS && !SWIGLU && (FMT != kF16 || MT >= 2)
+                          : FMT == kQ8_0 && MT == 2    ? (BLOCKS ? W == 8 && !SWIGLU : W == 8 || TN == 2)
+                          : BLOCKS                     ? MT == 1 && (FMT != kQ4_K || W == 8)
+                                                       : true;
 
 template <int FMT, int MT, int TN, int W, bool BLOCKS>
 hipError_t launch_scaled(const StreamArgs& a, std::uint32_t blocks, hipStream_t stream) {
     const dim3 threads(64 * (W + kProducers));
-    if constexpr (!kCompiled<FMT, MT, TN, W, BLOCKS>) {
-        return hipErrorInvalidConfiguration;
-    } else if (a.ffn_tiles == 0u) {
-        hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, false, false, BLOCKS>), dim3(blocks), threads, 0, stream, a);
-    } else if constexpr (dense_storage(FMT)) {
-        return hipErrorInvalidConfiguration;
-    } else if (a.serial > 1u) {
-        if constexpr (FMT == kQ8_0 && MT == 2 && W == 10) {
-            hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, true, true, false>), dim3(blocks), threads, 0, stream, a);
-        } else {
-            return hipErrorInvalidConfiguration;
+    const dim3 grid(blocks);
+    if (a.ffn_tiles == 0u) {
+        if constexpr (kReached<FMT, MT, TN, W, false, BLOCKS>) {
+            hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, false, false, BLOCKS>), grid, threads, 0, stream, a);
+            return hipGetLastError();
         }
-    } else {
-        hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, true, false, BLOCKS>), dim3(blocks), threads, 0, stream, a);
+    } else if (a.serial > 1u) {
+        if constexpr (FMT == kQ8_0 && MT == 2 && W == 10 && !BLOCKS) {
+            hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, true, true, false>), grid, threads, 0, stream, a);
+            return hipGetLastError();
+        }
+    } else if constexpr (kReached<FMT, MT, TN, W, true, BLOCKS>) {
+        hipLaunchKernelGGL((stream_kernel<FMT, MT, TN, W, true, false, BLOCKS>), grid, threads, 0, stream, a);
+        return hipGetLastError();
     }
-    return hipGetLastError();
+    return hipErrorInvalidConfiguration;
 }
 
 template <int FMT, int MT, int TN, int W>
