@@ -25,38 +25,42 @@
 //   * the activations come split under one power-of-two scale per row, or per
 //     (row, 32-block) where the kernel this one is taken instead of scaled
 //     blocks or steps (BLOCKS);
-//   * the K sum is formed in levels where registers allow (kLevels): pairs
-//     of steps, trips of the ring, then the total.  One running sum of the
-//     112 blocks of K = 3584 is 2.3e-7 from 64 bits (relative L2, Q8_0), the
-//     kernels this one replaces, whose waves split K, 1.6e-7, this one 1.5e-7.
+//   * the K sum is formed in levels where registers allow (kLevels says where,
+//     with the errors): pairs of steps, trips of the ring, then the total.
 //
-// What bounds it: HBM at one activation tile; at more, the L2 reads of the
-// activations (4 M K bytes per workgroup) and the LDS reads and VALU work per
-// weight tile, which grow with M.  Row tiles per workgroup are chosen so that
-// the grid is one round of the 256 CUs: a CU with two workgroups of eight
-// tiles finishes last (7B gate|up at 32 rows: 296 workgroups of eight tiles
-// 48 us, 237 of ten 36).
+// What bounds it (counters of 7B gate|up in profiles/decode_stream_sq_counters.md):
+// at one activation tile HBM (Q8_0 at 8 rows 144 MB in 32.5 us, 4.4 TB/s).  At more no
+// unit is full: at 64 rows VALU issue is at 33..47 % of its ceiling, the matrix
+// cores are busy 22..29 % of the time, LDS 28..35 % without a bank conflict,
+// and half of the wave time is waiting with three waves on a SIMD; time grows with
+// the instructions per weight tile, which grow with M.  Row tiles per workgroup
+// are chosen so that the grid is one round of the 256 CUs: a CU with two
+// workgroups of eight tiles finishes last (7B gate|up at 32 rows: 296 workgroups
+// of eight tiles 48 us, 237 of ten 36).
 //
-// Measured per linear (Qwen2-7B shapes, graph replay over copies larger than
-// the Infinity Cache, the split launch included; kernels replaced -> this):
+// Measured per linear (Qwen2-7B shapes, graph replay over copies of 320 MB or
+// more, the split launch included; kernels replaced -> this, both in one run;
+// - where the other kernel stays):
 //
 //                 M = 8           16            32            64
-//   gate|up Q8_0  34.6 -> 30.4    37.8 -> 30.7  (kept)        64.9 -> 52.7 us
-//           Q4_0  33.8 -> 23.1    35.0 -> 23.2  45.2 -> 31.8  66.6 -> 51.0
-//           Q4_K  38.4 -> 28.1    38.3 -> 28.9  51.9 -> 40.0  78.1 -> 60.7
-//   down    Q8_0  -               -             36.3 -> 33.8  47.1 -> 39.9
-//           Q4_0  -               -             34.7 -> 29.6  45.2 -> 38.6
-//           Q4_K  31.1 -> 25.5    32.0 -> 26.4  40.1 -> 32.3  51.8 -> 44.1
-//   q|k|v   Q8_0  -               -             18.2 -> 16.9  23.5 -> 21.7
-//   lm_head Q8_0  121 -> 107      123 -> 108    140 -> 121    195 -> 191
-//           Q4_0  91 -> 73        92 -> 78      126 -> 107    197 -> 169
-//           Q4_K  115 -> 89       112 -> 90     158 -> 130    253 -> 206
+//   gate|up Q8_0  38.2 -> 33.1    40.4 -> 33.4  -             64.4 -> 57.2 us
+//           Q4_0  34.9 -> 26.2    35.6 -> 26.7  45.6 -> 34.8  64.5 -> 51.7
+//           Q4_K  39.1 -> 30.7    39.0 -> 30.6  51.9 -> 40.9  79.4 -> 60.5
+//   down    Q8_0  -               -             36.5 -> 34.9  45.8 -> 43.7
+//           Q4_0  -               -             33.8 -> 31.8  43.1 -> 40.8
+//           Q4_K  31.4 -> 23.8    31.8 -> 24.5  39.4 -> 34.9  49.3 -> 45.6
+//   q|k|v   Q8_0  -               -             17.5 -> 17.2  23.6 -> 22.0
+//           Q4_0  -               -             16.5 -> 16.1  21.2 -> 21.5
+//           Q4_K  -               -             18.1 -> 17.8  24.5 -> 23.6
+//   lm_head Q8_0  123 -> 108      123 -> 111    138 -> 129    196 -> 184
+//           Q4_0  96 -> 78        97 -> 80      125 -> 111    194 -> 165
+//           Q4_K  124 -> 99       123 -> 98     156 -> 129    253 -> 202
 //
 // Dense rows (dense_mfma_kernel before, which asks for a Q6_K step in eight
 // 4-byte loads a lane; here a super-block is three 16-byte loads and its
-// scales): Q6_K down at 13 rows 63.8 -> 34.0, at 64 201 -> 60.4; gate|up 93.6
-// -> 43.2 and 255 -> 89.1; lm_head 331 -> 136 and 948 -> 327; F16 gate|up at 24
-// rows 99 -> 78.7, at 64 286 -> 90.3; down at 64 154 -> 62.9.
+// scales): Q6_K down at 13 rows 63.6 -> 30.4, at 64 200 -> 60.9; gate|up 91.7
+// -> 39.6 and 254 -> 97.6; lm_head 331 -> 139 and 949 -> 369; F16 gate|up at 24
+// rows 102 -> 79.1, at 64 287 -> 86.3; down 78.2 -> 50.9 and 154 -> 55.7.
 //
 // Replaces specialized_matmul_kernel / specialized_matmul_batch_reuse_kernel
 // (src/cuda/cuda_backend.cu:501-583) for batched decode.

@@ -345,7 +345,8 @@ hipError_t launch_wsplit_any(int type, const WsArgs& a, const WsplitShape& s, hi
 
 bool wsplit_preferred(const TilePlanes& p, std::uint32_t m) {
     // Measured against the skinny kernels on the Qwen2-7B shapes (graph
-    // replay, per linear; Q8_0 / Q4_0 / Q4_K at M = 8, 16, 32, 64):
+    // replay, per linear; Q8_0 / Q4_0 / Q4_K at M = 8, 16, 32, 64; the
+    // streaming kernel is asked first, stream_preferred):
     //  * one activation tile (M <= 16): faster on q|k|v, o, gate|up and
     //    down in every format (down 30.1 -> 23.6 us at M = 8 in Q8_0, gate|up
     //    39.3 -> 34.1, o 12.4 -> 10.7 at M = 16), except Q4_K q|k|v (even at

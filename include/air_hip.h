@@ -229,9 +229,11 @@ int air_hip_context_set_decode_pipeline(air_hip_context* ctx, uint32_t lds_stage
  * k_splits workgroups split K further (1..64, with a deterministic
  * reduction); split_x = 1 splits the activations into the workspace first,
  * 2 in each wave.  0 keeps the automatic choice.  Mode 0 takes the kernel
- * where it measured faster than the skinny kernels (every 7B matrix but the
- * lm_head at M <= 16, the narrow ones above) and only while the decode path
- * is automatic.  No counterpart in the reference. */
+ * where it measured faster than the skinny kernels and the streaming kernel
+ * does not run (of the 7B matrices q|k|v, o and down at M <= 16, in Q4_K only
+ * o; above, o and Q8_0 down up to 24 rows), and only while the decode path is
+ * automatic.  No counterpart
+ * in the reference. */
 int air_hip_context_set_wsplit(air_hip_context* ctx, uint32_t mode, uint32_t tile_n, uint32_t waves, uint32_t depth,
                                uint32_t k_splits, uint32_t split_x);
 /* Chooses the kernel of the dense matrices (F16, BF16 and Q6_K storage;
@@ -369,7 +371,7 @@ int air_hip_linear_plan(const air_hip_context* ctx, const air_hip_matrix* matrix
  * activations and K-split partials live in a 16 MiB device array per GPU,
  * and the one-row GEMV's pair-split row slots in a second one of 8192
  * words, both held from library load until the process ends (every
- * Qwen2-7B projection and lm_head at m <= 64 needs at most 12.5 MiB); a
+ * Qwen2-7B projection and lm_head at m <= 64 needs at most 12.8 MiB); a
  * linear needing more, m > 64, the PREFILL tactic, and the
  * fused kernel's cross-workgroup K split (a tuning override) return
  * AIR_HIP_UNSUPPORTED.  The array keeps the last call's contents and is
@@ -432,12 +434,15 @@ int air_hip_decode_linear_fused(air_hip_context* ctx, const air_hip_matrix* matr
  *     than k, in whole rows of the operand); a K split that carries the norm
  *     without it leaves the conversion to the next linear.
  * Bit-identical to air_hip_linear (same tactic) followed by that call.  Where
- * the linear runs with a K split (a skinny launch at decode widths 2..64,
- * or a prefill GEMM), its split reduction
- * applies the epilogue, so the epilogue costs no launch of its own; other
- * routes run the linear into a context buffer and the separate kernel.  out must not alias x.  No counterpart in the reference's
- * linear API: it replaces the executor's linear then add / SiLU sequence
- * (cuda_backend.cu:789, 849-860). */
+ * the linear runs with a K split (at decode widths 2..64, or a prefill GEMM),
+ * its split reduction applies the epilogue, and the streaming kernel applies
+ * SWIGLU itself where K is whole, so the epilogue costs no launch of its own;
+ * other routes run the linear into a context buffer and the separate kernel.
+ * SWIGLU over Q8_0 at 17..32 rows and 2000..4096 row tiles runs the streaming
+ * kernel too (both K splits in one workgroup), although air_hip_linear_plan,
+ * which describes the plain linear, names the skinny kernel there.  out must
+ * not alias x.  No counterpart in the reference's linear API: it replaces the
+ * executor's linear then add / SiLU sequence (cuda_backend.cu:789, 849-860). */
 int air_hip_linear_epilogue(air_hip_context* ctx, const air_hip_matrix* matrix, const float* x, uint32_t rows,
                             float* out, const float* bias, int epilogue, const float* norm_weight, float* norm_out,
                             double eps, int tactic);
