@@ -232,8 +232,7 @@ int air_hip_context_set_decode_pipeline(air_hip_context* ctx, uint32_t lds_stage
  * where it measured faster than the skinny kernels and the streaming kernel
  * does not run (of the 7B matrices q|k|v, o and down at M <= 16, in Q4_K only
  * o; above, o and Q8_0 down up to 24 rows), and only while the decode path is
- * automatic.  No counterpart
- * in the reference. */
+ * automatic.  No counterpart in the reference. */
 int air_hip_context_set_wsplit(air_hip_context* ctx, uint32_t mode, uint32_t tile_n, uint32_t waves, uint32_t depth,
                                uint32_t k_splits, uint32_t split_x);
 /* Chooses the kernel of the dense matrices (F16, BF16 and Q6_K storage;
@@ -365,7 +364,8 @@ int air_hip_linear_plan(const air_hip_context* ctx, const air_hip_matrix* matrix
  * so code under HIP graph capture, tight serving loops and harnesses that
  * forbid allocation can call it.  Same kernels and launch shapes as
  * air_hip_linear through this context (its tuning overrides included), so
- * the outputs are bit-identical; a K split that air_hip_linear sums inside
+ * the outputs are bit-identical (but for a captured air_hip_linear without its
+ * streaming buffers, air_hip_context_reserve); a K split that air_hip_linear sums inside
  * the kernel (air_hip_context_set_split_chain) takes the reduction launch
  * here, which the in-kernel sum reproduces bit for bit.  Its split
  * activations and K-split partials live in a 16 MiB device array per GPU,
