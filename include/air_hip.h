@@ -149,7 +149,8 @@ int air_hip_context_create(int device, void* stream, air_hip_context** out);
 int air_hip_context_destroy(air_hip_context* ctx);
 /* Rebinds the context to another stream, as cublasSetStream rebinds the
  * reference's handle (cuda_backend.cu:1780); work already queued stays on
- * the old one. */
+ * the old one and on the context's buffers, which the next calls use too:
+ * order the two streams first (an event, or a synchronize). */
 int air_hip_context_set_stream(air_hip_context* ctx, void* stream);
 /* Grows the workspaces so linears with input width <= max_k and up to max_m
  * rows never allocate on the hot path (workspace sizing,
