@@ -288,9 +288,9 @@ constexpr unsigned kLevels = FMT == kF16 && MT == 2 && TN == 2      ? 2u
 // that belong to them (TN = 2: both in one wave; else waves w and w + W / 2,
 // which meet in LDS), and it stores silu(gate) * up: the SwiGLU launch and
 // its round trip through the fused rows go away.  7B gate|up with its SwiGLU,
-// graph replay: at 32 rows Q8_0 46.2 -> 37.4 us (eight-wave kernel and its
-// reduction before), Q4_0 44.8 -> 32.3, Q4_K 51.0 -> 38.8; at 64 65.7 -> 54.7,
-// 67.6 -> 51.1, 81.4 -> 59.5 (the streaming kernel's share included).
+// graph replay: at 32 rows Q8_0 46.0 -> 38.7 us (eight-wave kernel and its
+// reduction before), Q4_0 44.4 -> 33.3, Q4_K 50.9 -> 39.7; at 64 67.2 -> 57.1,
+// 67.0 -> 50.9, 81.2 -> 60.1 (the streaming kernel's share included).
 // SERIAL: the K splits of a plan that sums them in a reduction, one after the
 // other in one workgroup: each in one running sum, scaled, then added from
 // zero in split order -- that plan's bits.
